@@ -11,14 +11,16 @@
 // Reference-compatible mode reproduces the stub exactly: dx = dy * gamma,
 // dgamma = dbeta = 0.
 //
-// Rows of up to 2048 columns whose width is a multiple of 32 (16-byte rows):
-// one launch, row blocks for dx beside (strip, chunk) blocks for
-// dgamma/dbeta (ln_bwd_onepass_kernel).  Other rows of up to 2048 columns:
+// The forward takes a wave per row up to 512 columns and a block per row
+// (ln_fwd_block_kernel) up to 16384.  The backward, for rows of up to 2048
+// columns whose width is a multiple of 32 (16-byte rows): one launch, row
+// blocks for dx beside (strip, chunk) blocks for dgamma/dbeta
+// (ln_bwd_onepass_kernel).  Other rows of up to 2048 columns:
 // one fused pass (one wave per row, the row held in registers; each wave
 // also accumulates its rows' dgamma/dbeta column partials, combined per block
 // in LDS and then across blocks by a fixed-order column-strip reduction).
-// Wider rows: a streaming row kernel for dx and a column kernel for
-// dgamma/dbeta.
+// 2049 to 16384 columns: a block per row (ln_bwd_block_kernel).  Wider rows:
+// streaming row kernels and a column kernel for dgamma/dbeta.
 #include "common.hpp"
 
 #include <algorithm>
@@ -458,6 +460,210 @@ __global__ __launch_bounds__(256) void ln_part_strip_kernel(const float* __restr
     }
 }
 
+// ---------------------------------------------------------------------------
+// A block of T threads per row, 4 * NC values a thread, so a row is read and
+// written once: forward from 513 columns, backward from 2049 (and from 1025
+// where the matrix is large), up to 16384.  Blocks walk rows b, b + grid, ...
+// and load the next row's values before the sums of the current one, so one
+// row's loads are in flight across the other's barriers and stores.
+// HBM-bound.  Measured with rotated buffers, before -> now:
+//   4096 x 8192: forward 164 -> 47 us (5.7 TB/s), backward 297 -> 75 us
+//     (5.35 TB/s of x, dy and dx), against streamed kernels that read a row
+//     two or three times with 4-byte loads;
+//   8192 x 1024: forward 26.3 -> 13.2 us, 1024 x 1024 5.9 -> 4.2 us, against
+//     a wave per row, whose 16 values a lane left too few loads in flight.
+// ---------------------------------------------------------------------------
+
+// Column of value (c, q) of this thread.
+template <int T, bool VEC>
+__device__ __forceinline__ int blk_col(int c, int q) {
+    return VEC ? 4 * (T * c + (int)threadIdx.x) + q : T * (4 * c + q) + (int)threadIdx.x;
+}
+
+template <int T, int NC, bool VEC, bool NT>
+__device__ __forceinline__ void blk_load(const float* __restrict__ row, int cols, float (&v)[NC][4]) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if constexpr (VEC) {
+            const int j = blk_col<T, true>(c, 0);
+            const float4 t = j < cols ? tfd::ld_v<NT>(reinterpret_cast<const float4*>(row + j))
+                                      : make_float4(0.f, 0.f, 0.f, 0.f);
+            v[c][0] = t.x; v[c][1] = t.y; v[c][2] = t.z; v[c][3] = t.w;
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = blk_col<T, false>(c, q);
+                v[c][q] = j < cols ? row[j] : 0.0f;
+            }
+        }
+    }
+}
+
+template <int T, int NC, bool VEC>
+__device__ __forceinline__ void blk_store(float* __restrict__ row, int cols, const float (&v)[NC][4]) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if constexpr (VEC) {
+            const int j = blk_col<T, true>(c, 0);
+            if (j < cols)
+                tfd::st_nt(reinterpret_cast<float4*>(row + j), make_float4(v[c][0], v[c][1], v[c][2], v[c][3]));
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int j = blk_col<T, false>(c, q);
+                if (j < cols) row[j] = v[c][q];
+            }
+        }
+    }
+}
+
+// Sum over the block: a butterfly per wave, the waves in order.  One barrier:
+// callers alternate between two `red` buffers, so a buffer is written again
+// only after the barrier that follows its last reads.
+template <int T>
+__device__ __forceinline__ float blk_sum(float v, float* red) {
+    v = tfd::wave_sum(v);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float s = red[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) s += red[w];
+    return s;
+}
+
+template <int T, int NC, bool VEC>
+__global__ __launch_bounds__(T) void ln_fwd_block_kernel(const float* __restrict__ x, const float* __restrict__ gamma,
+                                                         const float* __restrict__ beta, float* __restrict__ y,
+                                                         float* __restrict__ mean, float* __restrict__ rstd, int rows,
+                                                         int cols, float eps) {
+    __shared__ float red[2][T / 64];
+    const float inv_c = 1.0f / (float)cols;
+    float gm[NC][4], bt[NC][4], v[NC][4], next[NC][4];
+    blk_load<T, NC, VEC, false>(gamma, cols, gm);
+    blk_load<T, NC, VEC, false>(beta, cols, bt);
+    int r = blockIdx.x;
+    blk_load<T, NC, VEC, true>(x + (int64_t)r * cols, cols, next);
+    for (; r < rows; r += gridDim.x) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[c][q] = next[c][q];
+        if (r + (int)gridDim.x < rows) blk_load<T, NC, VEC, true>(x + (int64_t)(r + gridDim.x) * cols, cols, next);
+        float s = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) s += (v[c][0] + v[c][1]) + (v[c][2] + v[c][3]);
+        const float m = blk_sum<T>(s, red[0]) * inv_c;
+        float ss = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float d = blk_col<T, VEC>(c, q) < cols ? v[c][q] - m : 0.0f;
+                ss += d * d;
+            }
+        const float var = blk_sum<T>(ss, red[1]) * inv_c;
+        const float rs = 1.0f / sqrtf(var + eps);
+        if (threadIdx.x == 0) {
+            mean[r] = m;
+            rstd[r] = rs;
+        }
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[c][q] = (v[c][q] - m) * rs * gm[c][q] + bt[c][q];
+        blk_store<T, NC, VEC>(y + (int64_t)r * cols, cols, v);
+    }
+}
+
+// dx, and the block's column sums of dy * xhat and dy over its rows to
+// part[block][0][:] and part[block][1][:].
+template <int T, int NC, bool VEC>
+__global__ __launch_bounds__(T) void ln_bwd_block_kernel(const float* __restrict__ dy, const float* __restrict__ x,
+                                                         const float* __restrict__ gamma,
+                                                         const float* __restrict__ mean,
+                                                         const float* __restrict__ rstd, float* __restrict__ dx,
+                                                         float* __restrict__ part, int rows, int cols) {
+    __shared__ float red[2][2][T / 64];
+    // A block of 1024 threads has 128 registers a thread, too few for the
+    // next row (it spilled 36): the other waves cover its loads.
+    constexpr bool kAhead = T < 1024;
+    const float inv_c = 1.0f / (float)cols;
+    float gm[NC][4], gacc[NC][4], bacc[NC][4], xv[NC][4], gv[NC][4], xn[NC][4], gn[NC][4];
+    blk_load<T, NC, VEC, false>(gamma, cols, gm);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) gacc[c][q] = bacc[c][q] = 0.0f;
+    int r = blockIdx.x, turn = 0;
+    float m_next, rs_next;
+    auto load_next = [&](int row) __attribute__((always_inline)) {
+        blk_load<T, NC, VEC, true>(x + (int64_t)row * cols, cols, xn);
+        blk_load<T, NC, VEC, true>(dy + (int64_t)row * cols, cols, gn);
+        m_next = mean[row];
+        rs_next = rstd[row];
+    };
+    if (kAhead) load_next(r);
+    for (; r < rows; r += gridDim.x, turn ^= 1) {
+        if (!kAhead) load_next(r);
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                xv[c][q] = xn[c][q];
+                gv[c][q] = gn[c][q];
+            }
+        const float m = m_next, rs = rs_next;
+        if (kAhead && r + (int)gridDim.x < rows) load_next(r + (int)gridDim.x);
+        float s1 = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                // Past the last column gamma and dy are zero: no contribution.
+                const float xh = (xv[c][q] - m) * rs;
+                const float g = gv[c][q] * gm[c][q];
+                s1 += g;
+                s2 += g * xh;
+                gacc[c][q] += gv[c][q] * xh;
+                bacc[c][q] += gv[c][q];
+                xv[c][q] = xh;
+                gv[c][q] = g;
+            }
+        s1 = tfd::wave_sum(s1);
+        s2 = tfd::wave_sum(s2);
+        if ((threadIdx.x & 63) == 0) {
+            red[turn][0][threadIdx.x >> 6] = s1;
+            red[turn][1][threadIdx.x >> 6] = s2;
+        }
+        __syncthreads();
+        s1 = red[turn][0][0];
+        s2 = red[turn][1][0];
+#pragma unroll
+        for (int w = 1; w < T / 64; ++w) {
+            s1 += red[turn][0][w];
+            s2 += red[turn][1][w];
+        }
+        s1 *= inv_c;
+        s2 *= inv_c;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) xv[c][q] = rs * (gv[c][q] - s1 - xv[c][q] * s2);
+        blk_store<T, NC, VEC>(dx + (int64_t)r * cols, cols, xv);
+    }
+    float* pg = part + (int64_t)blockIdx.x * 2 * cols;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int j = blk_col<T, VEC>(c, q);
+            if (j < cols) {
+                pg[j] = gacc[c][q];
+                pg[cols + j] = bacc[c][q];
+            }
+        }
+}
+
 // Streaming dx for wide rows (three passes over the row).
 __global__ __launch_bounds__(256) void ln_bwd_dx_stream_kernel(const float* __restrict__ dy, const float* __restrict__ x,
                                                                const float* __restrict__ gamma,
@@ -534,6 +740,10 @@ int chunks_for(int64_t cols) {
 
 bool row_vec(const void* p, int64_t cols) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && cols % 4 == 0; }
 
+// Threads of the block-per-row kernels (four 16-byte groups a thread), or 0
+// where they do not take the width.
+int block_threads(int64_t cols) { return cols <= 4096 ? 256 : cols <= 8192 ? 512 : cols <= 16384 ? 1024 : 0; }
+
 int row_grid(int64_t rows) { return (int)std::min<int64_t>((rows + 3) / 4, 2048); }
 
 }  // namespace
@@ -548,11 +758,25 @@ tf_status tf_layernorm_fwd(tf_ctx* ctx, const float* x, const float* gamma, cons
     TF_REQUIRE(x && gamma && beta && y && mean && rstd, "tf_layernorm_fwd: null pointer");
     const int vec = row_vec(x, cols) && row_vec(y, cols);
     const dim3 grid(row_grid(rows));
+    if (const int t = cols > 512 ? block_threads(cols) : 0) {
+        const bool bvec = vec && row_vec(gamma, cols) && row_vec(beta, cols);
+        // Two blocks a CU of 512 threads and their like cover each row's
+        // barriers; narrow rows (one group of values a thread) want more.
+        const dim3 bgrid((unsigned)std::min<int64_t>(rows, (cols <= 1024 ? 524288 : 262144) / t));
+#define TF_LN_FWD(T, NC) \
+    if (bvec) ln_fwd_block_kernel<T, NC, true><<<bgrid, T, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps); \
+    else ln_fwd_block_kernel<T, NC, false><<<bgrid, T, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps)
+        if (cols <= 1024) { TF_LN_FWD(256, 1); }
+        else if (cols <= 2048) { TF_LN_FWD(256, 2); }
+        else if (t == 256) { TF_LN_FWD(256, 4); }
+        else if (t == 512) { TF_LN_FWD(512, 4); }
+        else { TF_LN_FWD(1024, 4); }
+#undef TF_LN_FWD
+        return tfh::check_launch("ln_fwd_block_kernel");
+    }
     switch (chunks_for(cols)) {
     case 1: ln_fwd_kernel<1><<<grid, 256, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps, vec); break;
     case 2: ln_fwd_kernel<2><<<grid, 256, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps, vec); break;
-    case 4: ln_fwd_kernel<4><<<grid, 256, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps, vec); break;
-    case kMaxCached: ln_fwd_kernel<kMaxCached><<<grid, 256, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps, vec); break;
     default: ln_fwd_stream_kernel<<<grid, 256, 0, ctx->stream>>>(x, gamma, beta, y, mean, rstd, (int)rows, (int)cols, eps); break;
     }
     return tfh::check_launch("ln_fwd_kernel");
@@ -581,7 +805,11 @@ tf_status tf_layernorm_bwd(tf_ctx* ctx, const float* dy, const float* x, const f
         if (st != TF_OK) return st;
         return tf_hip_fill_f32(ctx, dbeta, 0.0f, cols);
     }
-    const int nc = chunks_for(cols);
+    // Above 2^23 values (x and dy past 64 MB) the one-launch form's second
+    // read of x and dy by its column blocks comes from HBM again: 8192 x 2048
+    // takes 54.8 us with it, 40.5 us in a block a row; 8192 x 1024 23.4 and
+    // 24.2 us, 1024 x 1024 6.1 and 9.3 us.
+    const int nc = cols > 1024 && rows * cols > (int64_t(1) << 23) ? 0 : chunks_for(cols);
     const bool vec = row_vec(x, cols) && row_vec(dy, cols) && row_vec(dx, cols);
     const int64_t tstrips = cols / kLnStrip;
     if (nc > 0 && vec && cols % kLnStrip == 0 && tstrips <= tfh::kTicketColsumStrips) {
@@ -637,6 +865,32 @@ tf_status tf_layernorm_bwd(tf_ctx* ctx, const float* dy, const float* x, const f
         if (st != TF_OK) return st;
         // part is [nblocks][dgamma cols | dbeta cols]: column sums of a
         // [nblocks][2 cols] matrix, split into the two outputs.
+        const int64_t W = 2 * cols;
+        ln_part_strip_kernel<<<(unsigned)((W + 31) / 32), 256, 0, ctx->stream>>>(part, dgamma, dbeta, (int)nblocks,
+                                                                               (int)W, (int)cols, W % 4 == 0);
+        return tfh::check_launch("ln_part_strip_kernel");
+    }
+    if (const int t = block_threads(cols)) {
+        // A block a CU: the next row's loads are in flight beside a row's
+        // sums, and every block more adds a row of partials (2 x cols,
+        // written and read again): 4096 x 4096 takes 42.5 us on 256 blocks,
+        // 45.5 on 512; 333 x 5001 16.3 us on 128, 20.2 on 256.
+        const int64_t nblocks = std::min<int64_t>(rows, std::max<int64_t>(128, std::min<int64_t>(256, rows / 4)));
+        tf_status st = tfh::ensure_workspace(ctx, (size_t)nblocks * 2 * cols * sizeof(float));
+        if (st != TF_OK) return st;
+        float* part = reinterpret_cast<float*>(ctx->ws);
+        const bool bvec = vec && row_vec(gamma, cols);
+        const dim3 grid((unsigned)nblocks);
+#define TF_LN_BWD(T, NC) \
+    if (bvec) ln_bwd_block_kernel<T, NC, true><<<grid, T, 0, ctx->stream>>>(dy, x, gamma, mean, rstd, dx, part, (int)rows, (int)cols); \
+    else ln_bwd_block_kernel<T, NC, false><<<grid, T, 0, ctx->stream>>>(dy, x, gamma, mean, rstd, dx, part, (int)rows, (int)cols)
+        if (cols <= 2048) { TF_LN_BWD(256, 2); }
+        else if (t == 256) { TF_LN_BWD(256, 4); }
+        else if (t == 512) { TF_LN_BWD(512, 4); }
+        else { TF_LN_BWD(1024, 4); }
+#undef TF_LN_BWD
+        st = tfh::check_launch("ln_bwd_block_kernel");
+        if (st != TF_OK) return st;
         const int64_t W = 2 * cols;
         ln_part_strip_kernel<<<(unsigned)((W + 31) / 32), 256, 0, ctx->stream>>>(part, dgamma, dbeta, (int)nblocks,
                                                                                (int)W, (int)cols, W % 4 == 0);

@@ -48,6 +48,37 @@ def test_layernorm_fwd_bwd(ctx, R, Cc):
     assert_close(dbet.numpy(), want_db, RTOL32, "ln dbeta")
 
 
+# A block per row: the edges of its widths (513, 1024/1025, 2048/2049,
+# 4096/4097, 8192/8193, 16384/16385), rows of whole 16-byte groups and odd
+# ones, fewer rows than blocks and more, and the large narrow matrices whose
+# backward takes it too (rows * cols > 2^23).  rows, cols <= 2^15 terms a sum:
+# any fp32 order is within 2^15 * 2^-24 = 2e-3 of the sum of magnitudes in the
+# worst case and about sqrt of that (1e-5) here, so RTOL32 = 1e-4.
+@pytest.mark.parametrize("R,Cc", [(7, 513), (2100, 516), (5, 1025), (3, 2049), (700, 2052), (9, 4096), (300, 4097),
+                                  (2, 8192), (5, 8193), (1100, 5000), (3, 16384), (2, 16385), (8300, 1028),
+                                  (4300, 1999)])
+def test_layernorm_block_rows_vs_float64(ctx, R, Cc):
+    ops = _ops()
+    x, dy = synth.normal(211 + Cc, (R, Cc)) + np.float32(0.5), synth.normal(212 + Cc, (R, Cc))
+    gamma, beta = synth.normal(213, (Cc,), mean=1.0, std=0.1), synth.normal(214, (Cc,))
+    xd, g64 = x.astype(np.float64), dy.astype(np.float64) * gamma
+    m = xd.mean(1, keepdims=True)
+    rs = 1.0 / np.sqrt(((xd - m) ** 2).mean(1, keepdims=True) + 1e-5)
+    xh = (xd - m) * rs
+    dx_, dg_ = ctx.array(x), ctx.array(gamma)
+    y, mean, rstd = ctx.empty((R, Cc)), ctx.empty((R,)), ctx.empty((R,))
+    ops.layernorm_fwd(dx_, dg_, ctx.array(beta), y, mean, rstd)
+    assert_close(mean.numpy(), m[:, 0], RTOL32, "ln mean")
+    assert_close(rstd.numpy(), rs[:, 0], RTOL32, "ln rstd")
+    assert_close(y.numpy(), xh * gamma + beta, RTOL32, "ln fwd")
+    dx, dgam, dbet = ctx.empty((R, Cc)), ctx.empty((Cc,)), ctx.empty((Cc,))
+    ops.layernorm_bwd(ctx.array(dy), dx_, dg_, mean, rstd, dx, dgam, dbet)
+    want = rs * (g64 - g64.mean(1, keepdims=True) - xh * (g64 * xh).mean(1, keepdims=True))
+    assert_close(dx.numpy(), want, RTOL32, "ln dx")
+    assert_close(dgam.numpy(), (dy * xh).sum(0), RTOL32, "ln dgamma")
+    assert_close(dbet.numpy(), dy.astype(np.float64).sum(0), RTOL32, "ln dbeta")
+
+
 def test_layernorm_bwd_reference_stub_bitexact(ctx):
     ops = _ops()
     R, Cc = 1024, 1024
