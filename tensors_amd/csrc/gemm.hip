@@ -1946,6 +1946,36 @@ struct F32DlOperand {
 
 constexpr int kF32DlPairFloats = 8 * 8 * 64 * 4;  // LDS floats of the pair reduction (8 KB per wave)
 
+// Pair reduction through LDS of waves w and w ^ 4, which hold two k halves of
+// one 64 x 64 block: wave w hands sub-tile row block 1 - g to its partner and
+// keeps block g, complete (8 KB per wave, 1 KB per vector).  The caller has
+// synchronised the workgroup.
+__device__ __forceinline__ void pair_reduce(v16f (&acc)[2][2], int g, float* __restrict__ lds) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    f32x4* x = reinterpret_cast<f32x4*>(lds);
+    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
+        constexpr int i = decltype(I)::value;
+        if (i == g) return;
+        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
+            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
+            x[(wave * 8 + v) * 64 + lane] = f32x4{acc[i][j][r], acc[i][j][r + 1], acc[i][j][r + 2], acc[i][j][r + 3]};
+        });
+    });
+    __syncthreads();
+    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
+        constexpr int i = decltype(I)::value;
+        if (i != g) return;
+        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
+            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
+            const f32x4 y = x[((wave ^ 4) * 8 + v) * 64 + lane];
+            acc[i][j][r] += y[0];
+            acc[i][j][r + 1] += y[1];
+            acc[i][j][r + 2] += y[2];
+            acc[i][j][r + 3] += y[3];
+        });
+    });
+}
+
 // Epilogue of the direct fp32 kernel for interior blocks without beta * C or
 // a row bias.  The wave's 32 x 64 block (sub-tile row block g after the pair
 // reduction) is staged in its own 8 KB of LDS (`stage`, 32 rows x 64
@@ -2158,36 +2188,227 @@ __global__ __launch_bounds__(kF32DlThreads) void gemm_f32_dl_kernel(GemmParams p
         });
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the clamped loads
     }
-    // Pair reduction through LDS: wave w hands sub-tile row block 1 - g to
-    // wave w ^ 4 and keeps block g (8 KB per wave, 1 KB per vector).
     __syncthreads();  // every wave is done with the stages
-    f32x4* x = reinterpret_cast<f32x4*>(lds);
-    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
-        constexpr int i = decltype(I)::value;
-        if (i == g) return;
-        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
-            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
-            x[(wave * 8 + v) * 64 + lane] = f32x4{acc[i][j][r], acc[i][j][r + 1], acc[i][j][r + 2], acc[i][j][r + 3]};
-        });
-    });
-    __syncthreads();
-    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
-        constexpr int i = decltype(I)::value;
-        if (i != g) return;
-        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
-            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
-            const f32x4 y = x[((wave ^ 4) * 8 + v) * 64 + lane];
-            acc[i][j][r] += y[0];
-            acc[i][j][r + 1] += y[1];
-            acc[i][j][r + 2] += y[2];
-            acc[i][j][r + 3] += y[3];
-        });
-    });
+    pair_reduce(acc, g, lds);
     static_assert(kF32DlPairFloats + 8 * 32 * 64 <= S * 2 * kF32DlOp, "epilogue staging must fit in the ring");
     float* stage = lds + kF32DlPairFloats + wave * 32 * 64;  // past the pair-reduction area
     if (!f32dl_store_fast<!A_KMAJ, !B_KMAJ>(p, acc, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c,
                                             split, stage))
         store_wave<2, !A_KMAJ, !B_KMAJ>(p, acc, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split, g);
+}
+
+// ---------------------------------------------------------------------------
+// bf16 128 x 128 tiles for products with too few 256 x 256 tiles to fill the
+// GPU.  Operands go global -> LDS directly in 64-deep k blocks, a ring of
+// kMidStages blocks of 2 x 16 KB.  512 threads: waves w and w + 4 share a
+// 64 x 64 block (2 x 2 accumulators of v_mfma_f32_32x32x16_bf16) and take one
+// half of every k block each, so each SIMD runs two waves without the 64 x 32
+// blocks that would need 1.5 LDS fragment reads per MFMA instead of one; the
+// pair adds its halves through LDS at the end.
+//
+// One barrier per k block: passing the barrier of block t, every wave has
+// block t's fragments in registers and its share of block t + 1 has landed,
+// so block t's stage is refilled with block t + kMidStages and block t + 1's
+// fragments are read between block t's MFMAs.
+//
+// LDS layout of an operand block, written 1 KB per load instruction:
+//   K-major  [128 rows][64 k], 8 chunks of 16 bytes a row; chunk c of row r
+//            sits in slot c ^ ((r >> 1) & 7), so a b128 fragment read of 16
+//            rows hits all 64 banks once;
+//   MN-major [64 k][128 rows], chunk c of k row k in slot c ^ 4 (k % 4); read
+//            with ds_read_b64_tr_b16 as in DlOperand.
+// KTAIL: K % 64 != 0 (K % 8 == 0); loads at k >= K read zero.
+//
+// Bound by the loads into LDS: a 64-deep block takes 0.53 us (M = N = 2048,
+// K 2048 -> 8192), 0.51 without the MFMAs, 0.32 without the loads, 0.48 with
+// every workgroup loading one tile from a hot L2; its MFMAs alone need 0.21.
+// A fifth stage, and the loads issued together instead of between the
+// MFMAs, measured the same.  512 x 8192 x 4096: 820 TF/s.
+// ---------------------------------------------------------------------------
+constexpr int kMidTile = 128;
+constexpr int kMidK = 64;
+constexpr int kMidStages = 4;
+constexpr int kMidVec = kMidTile * kMidK * 2 / 16;      // u32x4 per operand block (16 KB)
+constexpr int kMidLoads = kMidVec * 16 / 1024 / 8;      // 1 KB loads per wave per operand block
+
+// Byte offsets of this lane's direct loads of an operand block, and their
+// first k within the block.
+template <bool KMAJ>
+__device__ __forceinline__ void mid_offsets(int64_t ld, uint32_t (&voff)[kMidLoads], int (&kl)[kMidLoads]) {
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < kMidLoads; ++i) {
+        const int blk = w * kMidLoads + i;
+        if (KMAJ) {
+            const int row = blk * 8 + (l >> 3);
+            kl[i] = 8 * ((l & 7) ^ ((row >> 1) & 7));
+            voff[i] = 2u * ((uint32_t)row * (uint32_t)ld + (uint32_t)kl[i]);
+        } else {
+            const int k = blk * 4 + (l >> 4);
+            kl[i] = k;
+            voff[i] = 2u * ((uint32_t)k * (uint32_t)ld + 8u * (uint32_t)((l & 15) ^ (4 * (k & 3))));
+        }
+    }
+}
+
+// Fragments of one operand: rows wbase + 32 i + l % 32 at k steps 2 g and
+// 2 g + 1 of a block (lane half h: k = 16 step + 8 h .. + 7).
+template <bool KMAJ>
+struct MidOperand {
+    int off[2];
+    __device__ __forceinline__ void init(int wbase, int g) {
+        const int l = threadIdx.x & 63, h = l >> 5;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (KMAJ) {
+                const int r = wbase + (l & 31);
+                off[s] = r * (kMidK / 8) + ((4 * g + 2 * s + h) ^ ((r >> 1) & 7));
+            } else {
+                const int q = l >> 4, a = l & 15, j = a >> 2;
+                const int m = wbase + 16 * (q & 1) + 4 * (a & 3);
+                off[s] = (32 * g + 16 * s + 8 * (q >> 1) + j) * kMidTile + (((m >> 3) ^ (4 * j)) * 8) + (m & 7);
+            }
+        }
+    }
+    // Sub-tile i adds 32 rows: the swizzles repeat every 16 (32) rows, so
+    // K-major it is a constant distance; MN-major the chunk index gains 4,
+    // which the rotation by 4 j turns into an exclusive or.
+    __device__ __forceinline__ v8bf frag(const u32x4* __restrict__ lds, int i, int s) const {
+        if constexpr (KMAJ) {
+            return __builtin_bit_cast(v8bf, lds[off[s] + i * 32 * (kMidK / 8)]);
+        } else {
+            const short* base = reinterpret_cast<const short*>(lds) + (off[s] ^ (32 * i));
+            const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)base);
+            const v4s hi =
+                __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(base + 4 * kMidTile));
+            return __builtin_bit_cast(v8bf, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+    }
+};
+
+struct MidFrags {
+    v8bf a[2][2], b[2][2];   // [k step][sub-tile]
+};
+
+template <bool A_KMAJ, bool B_KMAJ, bool KTAIL>
+__global__ __launch_bounds__(2 * kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_bf16_mid_kernel(GemmParams p) {
+    constexpr int S = kMidStages;
+    __shared__ u32x4 lds[S * 2 * kMidVec];
+    int tm, tn;
+    tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
+    const int split = blockIdx.y;
+    const int batch = blockIdx.z;
+    const int m0 = tm * kMidTile, n0 = tn * kMidTile;
+    const uint16_t* A = reinterpret_cast<const uint16_t*>(p.A) + (int64_t)batch * p.stride_a;
+    const uint16_t* B = reinterpret_cast<const uint16_t*>(p.B) + (int64_t)batch * p.stride_b;
+    const int kpb = KTAIL ? (p.K + kMidK - 1) / kMidK : p.K / kMidK;
+    const int kb_total = kpb * p.reduce_batch;
+    const int kb_beg = split * p.kb_per_split;
+    const int nk = max(0, min(kb_total, kb_beg + p.kb_per_split) - kb_beg);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int g = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+
+    v16f acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = v16f{};
+
+    if (nk > 0) {
+        MidOperand<A_KMAJ> oa;
+        MidOperand<B_KMAJ> ob;
+        oa.init(wm * 64, g);
+        ob.init(wn * 64, g);
+        uint32_t voff_a[kMidLoads], voff_b[kMidLoads];
+        int kl_a[kMidLoads], kl_b[kMidLoads];
+        mid_offsets<A_KMAJ>(p.lda, voff_a, kl_a);
+        mid_offsets<B_KMAJ>(p.ldb, voff_b, kl_b);
+        KWalk walk;
+        walk.init(A, B, 2 * p.stride_a, 2 * p.stride_b, kb_beg, nk, kpb);
+        const uint32_t ta0 = 2u * (A_KMAJ ? (uint32_t)m0 * (uint32_t)p.lda : (uint32_t)m0);
+        const uint32_t tb0 = 2u * (B_KMAJ ? (uint32_t)n0 * (uint32_t)p.ldb : (uint32_t)n0);
+        const uint32_t a_kstep = 2u * kMidK * (A_KMAJ ? 1u : (uint32_t)p.lda);
+        const uint32_t b_kstep = 2u * kMidK * (B_KMAJ ? 1u : (uint32_t)p.ldb);
+        const uint32_t wave_lds = lds_addr(lds) + dl_wave_offset<kMidLoads>();
+        // Load x (of 2 * kMidLoads) of the walk's next block into stage st.
+        auto issue = [&](int st, auto X) TF_LAMBDA_INLINE {
+            constexpr int x = decltype(X)::value, i = x % kMidLoads;
+            constexpr bool is_b = x >= kMidLoads;
+            const uint32_t dst = wave_lds + (uint32_t)(st * 2 * kMidVec * 16) + (is_b ? kMidVec * 16 : 0) + i * 1024u;
+            const uint32_t so = is_b ? tb0 + (uint32_t)walk.kin * b_kstep : ta0 + (uint32_t)walk.kin * a_kstep;
+            uint32_t v = is_b ? voff_b[i] : voff_a[i];
+            if constexpr (KTAIL) v = (is_b ? kl_b[i] : kl_a[i]) < p.K - walk.kin * kMidK ? v : kDlOob;
+            const uint32_t vv[1] = {v};
+            dl_issue<1>(is_b ? dl_rsrc(walk.b_base, p.b_bytes) : dl_rsrc(walk.a_base, p.a_bytes), so, vv, dst);
+        };
+        auto read = [&](int st, MidFrags& f) TF_LAMBDA_INLINE {
+            const u32x4* la = lds + st * 2 * kMidVec;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) f.a[s][i] = oa.frag(la, i, s);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) f.b[s][j] = ob.frag(la + kMidVec, j, s);
+            }
+        };
+        // A quarter of a block's MFMAs: k step q / 2, sub-tile row q % 2.
+        auto mfma = [&](const MidFrags& f, auto Q) TF_LAMBDA_INLINE {
+            constexpr int s = decltype(Q)::value >> 1, i = decltype(Q)::value & 1;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.a[s][i], f.b[s][j], acc[i][j], 0, 0, 0);
+        };
+        // A quarter of a block's fragment reads: k step q / 2, A's or B's.
+        auto read_q = [&](int st, MidFrags& f, auto Q) TF_LAMBDA_INLINE {
+            constexpr int s = decltype(Q)::value >> 1;
+            const u32x4* la = lds + st * 2 * kMidVec;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if constexpr ((decltype(Q)::value & 1) == 0) f.a[s][i] = oa.frag(la, i, s);
+                else f.b[s][i] = ob.frag(la + kMidVec, i, s);
+            }
+        };
+        MidFrags f[2];
+        // Prologue: blocks 0 .. S-1 (clamped) into stages 0 .. S-1.
+        static_for<S>([&](auto Bc) TF_LAMBDA_INLINE {
+            static_for<2 * kMidLoads>([&](auto X) TF_LAMBDA_INLINE { issue(decltype(Bc)::value, X); });
+            walk.advance();
+        });
+        dl_barrier<(S - 1) * 2 * kMidLoads>();
+        read(0, f[0]);
+        int t = 0, st = 0;
+        bool stop = false;
+        while (!stop) {
+            static_for<2>([&](auto Pc) TF_LAMBDA_INLINE {
+                constexpr int cur = decltype(Pc)::value;
+                if (stop) return;
+                // This wave's share of block t + 1 has landed (the newer
+                // S - 2 blocks may be in flight) and its reads of block t.
+                dl_barrier<(S - 2) * 2 * kMidLoads>();
+                const int next = st + 1 == S ? 0 : st + 1;
+                static_for<4>([&](auto Q) TF_LAMBDA_INLINE {
+                    read_q(next, f[1 - cur], Q);           // unused after the last block
+                    mfma(f[cur], Q);
+                    issue(st, Q);                          // of block min(t + S, nk - 1)
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                walk.advance();
+                st = next;
+                ++t;
+                if (t >= nk) stop = true;
+            });
+        }
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the clamped loads
+    }
+    __syncthreads();  // every wave is done with the stages
+    float* sf = reinterpret_cast<float*>(lds);
+    pair_reduce(acc, g, sf);
+    static_assert(kF32DlPairFloats + 8 * 32 * 64 <= S * 2 * kMidVec * 4, "epilogue staging must fit in the ring");
+    float* stage = sf + kF32DlPairFloats + wave * 32 * 64;
+    if (!f32dl_store_fast<false, false>(p, acc, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split,
+                                        stage))
+        store_wave<2, false, false>(p, acc, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split, g);
 }
 
 // Small fp32 products (C1's layers, C4's fully connected layer): one block
@@ -2808,6 +3029,19 @@ KernelFn pick_bf16_dl(bool a_kmaj, bool b_kmaj, bool ktail) {
     }
 }
 
+KernelFn pick_bf16_mid(bool a_kmaj, bool b_kmaj, bool ktail) {
+    if (ktail) {
+        if (a_kmaj && b_kmaj) return gemm_bf16_mid_kernel<true, true, true>;
+        if (a_kmaj && !b_kmaj) return gemm_bf16_mid_kernel<true, false, true>;
+        if (!a_kmaj && b_kmaj) return gemm_bf16_mid_kernel<false, true, true>;
+        return gemm_bf16_mid_kernel<false, false, true>;
+    }
+    if (a_kmaj && b_kmaj) return gemm_bf16_mid_kernel<true, true, false>;
+    if (a_kmaj && !b_kmaj) return gemm_bf16_mid_kernel<true, false, false>;
+    if (!a_kmaj && b_kmaj) return gemm_bf16_mid_kernel<false, true, false>;
+    return gemm_bf16_mid_kernel<false, false, false>;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // Split count for a grid of `tiles` workgroups over `kblocks` k blocks:
@@ -2868,6 +3102,47 @@ tf_status partials_buffer(tf_ctx* ctx, size_t need, bool noalloc, float** out) {
     return TF_OK;
 }
 
+// Which direct-to-LDS kernel runs a bf16 product, and over how many K
+// slices: the one with the smaller estimated time.  Both put one workgroup on
+// a CU, so a product takes whole rounds of `ncu` tiles; measured over
+// products of 256 to 4096 rows, N(0, 1) operands and K from 512 to 8192 (us):
+//   256 x 256 tiles: 12 + 0.0255 K a round (4096 x 4096 x 1000 36-41,
+//     x 4096 108-118), 128 x 128 tiles: 4.4 + 0.0083 K (2048 x 2048 x 2048
+//     21-24, x 8192 72-79): a quarter of the tile at a third of the time a k
+//     step, bound by the loads into LDS;
+//   a K split: 4.5 and 0.2 a MB of partials (the 128 tiles 0.4: their
+//     kernel's own stores are of the same order as its k loop).
+// So the large tiles stay for products that fill the GPU with them, and
+// 512 x 8192 x 4096 goes 58 -> 42 us, 512 x 4096 x 8192 131-255 -> 50,
+// 4096 x 1000 x 4096 53 -> 40, 2048 x 2048 x 2048 41 -> 22, 1024 x 1024 x
+// 1024 21-24 -> 12.
+struct Bf16Plan {
+    bool big;
+    int splits;
+};
+Bf16Plan bf16_plan(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t batch, bool big_fits, int big_splits,
+                   size_t partial_limit) {
+    const double mb = (double)M * (double)N * 4e-6;   // MB of one slice's partials
+    auto tiles = [&](int64_t t) { return ((M + t - 1) / t) * ((N + t - 1) / t) * batch; };
+    auto rounds = [&](int64_t t, int s) { return (double)((tiles(t) * s + ncu - 1) / ncu); };
+    Bf16Plan best{false, 1};
+    double least = rounds(kMidTile, 1) * (4.4 + 0.0083 * (double)K);
+    for (const int s : {2, 3, 4, 6, 8, 12, 16, 24, 32}) {
+        if (batch > 1 || s * 2 * kMidK > K || (size_t)s * (size_t)M * (size_t)N * 4 > partial_limit) break;
+        const double t = rounds(kMidTile, s) * (4.4 + 0.0083 * (double)K / s) + 4.5 + 0.4 * mb * s;
+        if (t < least) {
+            least = t;
+            best.splits = s;
+        }
+    }
+    if (big_fits) {
+        const double t = rounds(kBigTile, big_splits) * (12.0 + 0.0255 * (double)K / big_splits) +
+                         (big_splits > 1 ? 4.5 + 0.2 * mb * big_splits : 0.0);
+        if (t <= least) best = Bf16Plan{true, big_splits};
+    }
+    return best;
+}
+
 // Grid of the small-product kernel for an M x N x K product: 32 x 32 tiles
 // and enough chunk groups for ~256 blocks, at most 32 per tile (the last
 // block adds them up), each of >= 1 chunk of 64 k.  False when the product
@@ -2923,7 +3198,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     const int64_t ncu = ctx->num_cus;
     // bf16 with enough work for one 256 x 256 tile per CU (directly, or with
     // K split over at most 4 slices of >= 8 k blocks): the large-tile kernel.
-    bool big = false;
+    bool big = false, mid = false;
     int splits = 1;
     if (in_dtype == TF_BF16 && M >= 128 && N >= 128) {
         const int64_t tb = ((M + kBigTile - 1) / kBigTile) * ((N + kBigTile - 1) / kBigTile) * grid_batch;
@@ -2934,6 +3209,28 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
             splits = s;
         }
     }
+    // tf_gemm_noalloc takes the products whose large-tile split fits its
+    // scratch, whichever kernel then runs them.
+    if (noalloc && splits > 1) {
+        float* unused = nullptr;
+        tf_status st = partials_buffer(ctx, (size_t)splits * (size_t)M * (size_t)N * sizeof(float), noalloc, &unused);
+        if (st != TF_OK) return st;
+    }
+    // The direct-to-LDS kernels need 16-byte loadable operands, a K of whole
+    // 16-byte loads and extents that fit the buffer descriptor (taken as int).
+    const int64_t ext_a = trans_a ? (K - 1) * lda + M : (M - 1) * lda + K;
+    const int64_t ext_b = trans_b ? (N - 1) * ldb + K : (K - 1) * ldb + N;
+    const bool ext_ok = ext_a * esz <= (int64_t)0x7fffffff && ext_b * esz <= (int64_t)0x7fffffff;
+    p.vec_a = aligned16(A) && (lda % vec_elems == 0) && (stride_a % vec_elems == 0);
+    p.vec_b = aligned16(B) && (ldb % vec_elems == 0) && (stride_b % vec_elems == 0);
+    if (in_dtype == TF_BF16 && K > 0 && K % 8 == 0 && p.vec_a && p.vec_b && ext_ok && (trans_a == 0 || M % 8 == 0) &&
+        (trans_b != 0 || N % 8 == 0)) {
+        const Bf16Plan plan = bf16_plan(ncu, M, N, K * (reduce_batch ? batch : 1), grid_batch, big, splits,
+                                        noalloc ? kNoAllocScratchBytes : ~size_t(0));
+        big = plan.big;
+        mid = !plan.big;
+        splits = plan.splits;
+    }
     // Otherwise: tile width 128 x 128 when that gives every CU at least its
     // resident workgroup count (fp32: one, its three LDS stages take 108 KB;
     // bf16: two, which hide each other's barrier and LDS latency), 128 x 64
@@ -2941,14 +3238,12 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     const int64_t per_cu = in_dtype == TF_F32 ? 1 : 2;
     const int64_t tiles_m = big ? (M + kBigTile - 1) / kBigTile : (M + BM - 1) / BM;
     const int64_t t128 = tiles_m * ((N + 127) / 128) * grid_batch;
-    const int BN = big ? kBigTile : (N <= 64 || t128 < per_cu * ncu) ? 64 : 128;
+    const int BN = big ? kBigTile : mid ? 128 : (N <= 64 || t128 < per_cu * ncu) ? 64 : 128;
     p.tiles_m = (int)tiles_m;
     p.tiles_n = (int)((N + BN - 1) / BN);
     p.alpha = alpha; p.beta = beta; p.epi = epi; p.row_bias = row_bias;
     p.out_bf16 = out_dtype == TF_BF16;
     p.reduce_batch = reduce_batch ? (int)batch : 1;
-    p.vec_a = aligned16(A) && (lda % vec_elems == 0) && (stride_a % vec_elems == 0);
-    p.vec_b = aligned16(B) && (ldb % vec_elems == 0) && (stride_b % vec_elems == 0);
     p.mask_a = mask_a;
     if (mask_a && !aligned16(mask_a)) p.vec_a = 0;
     p.pair_c = (reinterpret_cast<uintptr_t>(C) & 7) == 0 && (ldc % 2 == 0) && (p.stride_c % 2 == 0);
@@ -3014,17 +3309,18 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         gemm_f32_smallk_kernel<<<grid, 256, 0, ctx->stream>>>(p);
         return tfh::check_launch("gemm_f32_smallk_kernel");
     }
+    if (mid) {
+        p.a_bytes = (uint32_t)(ext_a * esz);
+        p.b_bytes = (uint32_t)(ext_b * esz);
+    }
     if (big) {
         // Interior tiles take the direct-to-LDS kernel when the operands are
         // 16-byte loadable, K is a whole number of 16-byte loads (both
         // kernels count splits in 64-deep blocks, the last one partial when
         // K % 64 != 0, so their split boundaries agree) and each operand's
         // extent fits the buffer descriptor.
-        const int64_t ext_a = trans_a ? (K - 1) * lda + M : (M - 1) * lda + K;
-        const int64_t ext_b = trans_b ? (N - 1) * ldb + K : (K - 1) * ldb + N;
-        const int64_t lim = (int64_t)0x7fffffff;  // descriptor extent is passed as int
         const int64_t k_unit = kBf16Kernel >= 1 ? 8 : 64;   // the four-wave kernel has no K tail
-        const bool direct = K > 0 && K % k_unit == 0 && p.vec_a && p.vec_b && ext_a * esz <= lim && ext_b * esz <= lim;
+        const bool direct = K > 0 && K % k_unit == 0 && p.vec_a && p.vec_b && ext_ok;
         p.a_bytes = direct ? (uint32_t)(ext_a * esz) : 0u;
         p.b_bytes = direct ? (uint32_t)(ext_b * esz) : 0u;
         // Partial tiles at the M / N edges are fine for the direct kernel:
@@ -3045,10 +3341,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     // an MN-major operand needs its row count a multiple of 4 for that.
     bool dl32 = false;
     if (in_dtype == TF_F32 && BN == 128) {
-        const int64_t ext_a = trans_a ? (K - 1) * lda + M : (M - 1) * lda + K;
-        const int64_t ext_b = trans_b ? (N - 1) * ldb + K : (K - 1) * ldb + N;
-        const int64_t lim = (int64_t)0x7fffffff;
-        if (K > 0 && K % 32 == 0 && p.vec_a && p.vec_b && ext_a * 4 <= lim && ext_b * 4 <= lim) {
+        if (K > 0 && K % 32 == 0 && p.vec_a && p.vec_b && ext_ok) {
             const bool part_m = trans_a == 0 || M % 4 == 0;
             const bool part_n = trans_b != 0 || N % 4 == 0;
             p.int_m = part_m ? p.tiles_m : (int)(M / BM);
@@ -3066,7 +3359,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     // Split the k blocks when the tiles leave most CUs idle and K is long
     // (target: the resident workgroups of every CU, >= 4 k blocks per slice).
     const int64_t kblocks = ((K + BK - 1) / BK) * p.reduce_batch;
-    if (!big && grid_batch == 1 && tiles * 2 <= ncu && kblocks >= 8)
+    if (!big && !mid && grid_batch == 1 && tiles * 2 <= ncu && kblocks >= 8)
         splits = choose_splits(tiles, kblocks, per_cu * ncu, 4);
     if (kblocks == 0) {
         splits = 1;
@@ -3103,6 +3396,11 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
             st = tfh::check_launch("gemm_bf16_big_kernel");
             if (st != TF_OK) return st;
         }
+    } else if (mid) {
+        dim3 grid((unsigned)tiles, (unsigned)splits, (unsigned)grid_batch);
+        pick_bf16_mid(a_kmaj, b_kmaj, K % 64 != 0)<<<grid, 2 * kThreads, 0, ctx->stream>>>(p);
+        st = tfh::check_launch("gemm_bf16_mid_kernel");
+        if (st != TF_OK) return st;
     } else if (dl32) {
         const int64_t n_int = (int64_t)p.int_m * p.int_n;
         GemmParams q = p;

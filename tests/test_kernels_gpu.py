@@ -488,6 +488,51 @@ def test_gemm_bf16_direct_k_tail(ctx, ta, tb, nb, M, N, K, pad):
     assert_close(dc.numpy(), truth, RTOL16, f"bf16 K tail ta={ta} tb={tb} {nb}x{M}x{N}x{K} pad={pad}")
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("nb,reduce,M,N,K,pad,epi,out_bf16,beta", [
+    (1, False, 128, 128, 64, 0, "none", False, 0.0),          # one tile, one k block
+    (1, False, 8, 16, 8, 8, "bias_relu", False, 0.0),         # a corner of one tile, 56 of 64 k masked
+    (1, False, 136, 264, 136, 0, "bias", True, 0.0),          # ragged edges and K tail
+    (1, False, 120, 384, 320, 8, "none", False, 0.5),         # beta * C; more blocks than ring stages
+    (1, False, 248, 256, 2048, 0, "row_bias_relu", False, 0.0),  # K split over slices
+    (3, False, 136, 128, 200, 8, "row_bias", True, 0.0),      # independent products
+    (5, True, 128, 200, 72, 8, "none", False, 0.0),           # batch reduction: the walk wraps after a tail
+])
+def test_gemm_bf16_mid_tile(ctx, ta, tb, nb, reduce, M, N, K, pad, epi, out_bf16, beta):
+    """The 128 x 128 bf16 tiles at the edges of their tile, ring and walk.
+    The products of bf16 values are exact in fp32 and their sums of up to 2048
+    terms are off by at most 2048 * 2^-24 = 1.2e-4 of the sum of magnitudes,
+    about 1e-5 here: RTOL32, and one bf16 rounding (2^-8) more where C is
+    bf16.  Past K and the row ends lie values that would show in the sums."""
+    import tensors_amd as ta_mod
+    from tensors_amd import _lib, ops
+    lda, ldb = (M if ta else K) + pad, (K if tb else N) + pad
+    a_shape, b_shape = (nb, K if ta else M, lda), (nb, N if tb else K, ldb)
+    a16 = ta_mod.f32_to_bf16_bits(synth.normal(261 + K, a_shape))
+    b16 = ta_mod.f32_to_bf16_bits(synth.normal(262 + K, b_shape))
+    a, b = ta_mod.bf16_bits_to_f32(a16), ta_mod.bf16_bits_to_f32(b16)
+    c0 = synth.normal(263, (1 if reduce else nb, M, N))
+    dc = ctx.zeros(c0.shape, ta_mod.BF16) if out_bf16 else ctx.array(c0)
+    rows = epi.startswith("row")
+    bias = None if epi == "none" else synth.normal(264, (M if rows else N,))
+    code = {"none": _lib.TF_EPI_NONE, "bias": _lib.TF_EPI_BIAS, "bias_relu": _lib.TF_EPI_BIAS_RELU,
+            "row_bias": _lib.TF_EPI_ROW_BIAS, "row_bias_relu": _lib.TF_EPI_ROW_BIAS_RELU}[epi]
+    ops.gemm_ex(ctx.array(a16, ta_mod.BF16), ctx.array(b16, ta_mod.BF16), dc, M, N, K, lda=lda, ldb=ldb, ldc=N,
+                trans_a=ta, trans_b=tb, stride_a=a_shape[1] * lda, stride_b=b_shape[1] * ldb, stride_c=M * N, batch=nb,
+                reduce_batch=reduce, alpha=0.75, beta=beta, epilogue=code,
+                bias=None if bias is None else ctx.array(bias))
+    prod = [_gemm_truth(a[e][:, :M] if ta else a[e][:, :K], b[e][:, :K] if tb else b[e][:, :N], ta, tb)
+            for e in range(nb)]
+    truth = 0.75 * (sum(prod)[None] if reduce else np.stack(prod)) + beta * c0.astype(np.float64)
+    if bias is not None:
+        truth = truth + (bias[:, None] if rows else bias[None, :]).astype(np.float64)
+    if epi.endswith("relu"):
+        truth = np.maximum(truth, 0.0)
+    got = dc.numpy()
+    got = ta_mod.bf16_bits_to_f32(got) if out_bf16 else got
+    assert_close(got, truth, 2.0 ** -8 if out_bf16 else RTOL32, f"bf16 128 tile {nb}x{M}x{N}x{K} {epi}")
+
+
 @pytest.mark.parametrize("M,N,K,nb,shared_a,epi,out_bf16,beta", [
     (32, 1024, 27, 4, True, "row_bias_relu", False, 0.0),   # convolution over 3 channels, 3x3
     (64, 300, 32, 2, False, "bias", False, 0.0),            # ragged N, column bias, A per element
