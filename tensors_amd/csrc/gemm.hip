@@ -20,13 +20,13 @@
 // the reference's sequential loop (tensor/Tensor.cpp:356-360) within fp32
 // tolerance.
 //
-// fp32 tile: 128 x BN x 32 per 256-thread workgroup, BN = 128 or 64 (4 waves
-// in 2 x 2, each wave 64 x BN/2 = 2 x BN/64 tiles of v_mfma_f32_32x32x2_f32),
-// LDS double buffered with one barrier per k block, global loads for block
-// k+1 issued before the MFMAs of block k; interior tiles take an unguarded
-// 16-byte load path.  bf16: same structure with v_mfma_f32_32x32x16_bf16 and
-// a 64-deep k block.  At most ~74 KB of LDS per workgroup, so two workgroups
-// share a CU and fill each other's stalls.
+// Kernels, by what the operands allow: direct-to-LDS tiles (bf16 256 x 256 and
+// 128 x 128; fp32 128 x 128, 128 x 64 and 64 x 128, any alignment) with the
+// choice between them in bf16_plan and f32_plan; one-launch kernels for small
+// and narrow fp32 products; and register-staged tiles of 128 x 128 or
+// 128 x 64 (4 waves in 2 x 2, LDS double buffered, bounds-checked loads) for
+// the rest: bf16 operands that are not 16-byte loadable, and extents past
+// 2 GB.
 //
 // Work distribution: the tile index is remapped so that each of the 8 XCDs
 // (which receive workgroups round-robin) owns a contiguous, row-grouped block
@@ -90,16 +90,15 @@ struct GemmParams {
     int vec_c4;            // 4-element vector stores legal for C (16 bytes fp32, 8 bytes bf16)
     uint32_t a_bytes, b_bytes;  // byte extent of one batch element of A / B (buffer loads)
     int int_m, int_n;           // large-tile path: tile rows / columns covered by the direct kernel
+    unsigned* tickets;          // arrival counters by tile (products split by units)
+    int units_tile;             // k blocks of a tile; every workgroup takes units_per of the tiles'
+    int units_per, units_rem;   // k blocks, the first units_rem one more
     const float* mask_a;        // small fp32 path: A(m, k) taken as A(m, k) * (mask(m, k) > 0), mask laid out as A
 };
 
-// Remap a linear workgroup id so that the ids one XCD receives (id % 8 == x)
-// cover a contiguous range of tiles, then order tiles in groups of GROUP_M
-// tile-rows so concurrently running workgroups share A and B panels.
-__device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
-    const int total = tiles_m * tiles_n;
-    int id = wg;
-    if ((total & 7) == 0) id = (wg & 7) * (total >> 3) + (wg >> 3);
+// Tile `id` of a tiles_m x tiles_n grid taken in groups of four tile rows,
+// column by column.
+__device__ __forceinline__ void grouped_tile(int id, int tiles_m, int tiles_n, int& tm, int& tn) {
     constexpr int GROUP_M = 4;
     const int group_size = GROUP_M * tiles_n;
     const int g = id / group_size;
@@ -108,6 +107,16 @@ __device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, in
     const int in_g = id - g * group_size;
     tm = first_m + in_g % gm;
     tn = in_g / gm;
+}
+
+// Remap a linear workgroup id so that the ids one XCD receives (id % 8 == x)
+// cover a contiguous range of tiles, then order tiles in groups of GROUP_M
+// tile-rows so concurrently running workgroups share A and B panels.
+__device__ __forceinline__ void tile_coords(int wg, int tiles_m, int tiles_n, int& tm, int& tn) {
+    const int total = tiles_m * tiles_n;
+    int id = wg;
+    if ((total & 7) == 0) id = (wg & 7) * (total >> 3) + (wg >> 3);
+    grouped_tile(id, tiles_m, tiles_n, tm, tn);
 }
 
 // Tile of an edge-kernel workgroup.  With an interior grid of int_m x int_n
@@ -1585,7 +1594,8 @@ void gemm_bf16_big_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 kernel: 128 x BN x 32 per 256-thread workgroup (BN = 128, or 64 for
+// fp32 kernel for operands the direct-to-LDS kernels cannot describe (extents
+// past 2 GB): 128 x BN x 32 per 256-thread workgroup (BN = 128, or 64 for
 // grids that would leave CUs idle), 4 waves in 2 x 2, each 64 x BN/2 =
 // 2 x NSUB accumulators of v_mfma_f32_32x32x2_f32.
 //
@@ -1832,241 +1842,591 @@ __global__ __launch_bounds__(kThreads) void gemm_f32_kernel(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 direct-to-LDS kernel (tiles inside an int_m x int_n grid of 128 x 128,
-// K % 32 == 0, 16-byte loadable operands): the global loads write LDS
-// directly (buffer_load_dwordx4 ... lds, as in the bf16 direct kernel), so no
-// staging registers and no LDS stores; block k's loads are issued two blocks
-// ahead into a four-stage ring (128 KB).
+// fp32 direct-to-LDS kernel: the global loads write LDS directly
+// (buffer_load ... lds, as in the bf16 direct kernel), so no staging
+// registers and no LDS stores; block k's loads are issued two blocks ahead
+// into a ring of 32-deep k blocks.
 //
-// 512 threads: waves w and w + 4 share the 64 x 64 output block w & 3 (2 x 2
-// sub-tiles of v_mfma_f32_32x32x2_f32) and split every 32-deep block: group
-// g = w / 4 takes quads 2g and 2g + 1 (lane half h feeds k = 16h + 4q + s at
-// step s of quad q, the k order of the register-staged kernel).  Two waves
-// per SIMD keep its matrix core busy through each other's barrier and LDS
-// waits.  At the end each pair adds its halves through LDS (own + partner:
-// the same sum in both waves, fp addition commutes) and each wave stores one
-// 32-row sub-tile of the block.
+// Tiles of 64 MI x 64 NI (MI, NI = 1 or 2, not both 1).  512 threads: waves w
+// and w + 4 share the 32 MI x 32 NI output block w & 3 (MI x NI sub-tiles of
+// v_mfma_f32_32x32x2_f32) and split every 32-deep block: group g = w / 4
+// takes quads 2g and 2g + 1 (lane half h feeds k = 16h + 4q + s at step s of
+// quad q, the k order of the register-staged kernel).  Two waves per SIMD
+// keep its matrix core busy through each other's barrier and LDS waits.  At
+// the end each pair adds its halves through LDS (own + partner: the same sum
+// in both waves, fp addition commutes) and each wave stores one half of the
+// block.
 //
-// LDS layout per operand block (16 KB, written 1 KB per load instruction):
-//   K-major  [128 rows][8 chunks of 4 k]; chunk c of row r sits in slot
+// LDS layout per operand block (R = 128 or 64 rows):
+//   K-major  [R rows][8 chunks of 4 k]; chunk c of row r sits in slot
 //            c ^ f32dl_swz(r), so the b128 fragment reads of 16 consecutive
 //            rows hit 16 distinct 4-bank groups (rows 2 apart share banks);
-//   MN-major [32 k][128 rows], as in memory; a lane reads the row pair
-//            2c, 2c + 1 of one k with one ds_read_b64, so sub-tile 0 of a
+//   MN-major [32 k][R rows], as in memory; with R = 128 a lane reads the row
+//            pair 2c, 2c + 1 of one k with one ds_read_b64, so sub-tile 0 of a
 //            wave holds its rows 2c and sub-tile 1 its rows 2c + 1 (the
 //            epilogue writes those rows / columns interleaved).
+//
+// MODE: how the loads fill a block.
+//   kF32Whole 16-byte loads, K % 32 == 0 (gemm_f32_whole_kernel);
+//   kF32Tail  16-byte loads, K a whole number of them where it is a row;
+//   kF32Words 4-byte loads: any K, leading dimension and row count.
+// The last two give a load of k >= K an offset past the descriptor, so it
+// reads zero (a compare and a select a load).  Four times as many load
+// instructions cost little here: a 128 x 128 block takes 4096 MFMA cycles per
+// SIMD and 128 load instructions per CU.
+//
+// Work split.  The product's units are (tile, k block) pairs, tile by tile;
+// workgroup w takes units start(w) .. start(w + 1) - 1 of an even split
+// (GemmParams::units_per, units_rem), one tile segment after the other.  With
+// as many workgroups as tiles that is one whole tile each; with one workgroup
+// per resident slot instead, a product whose tiles do not come in whole
+// rounds still keeps every CU busy to the end, and one with few tiles splits
+// its k range evenly.  A tile that several workgroups share is added by the
+// last of them to arrive: each stores its partial tile (in register order, so
+// the stores and loads are whole lines) with agent-scope stores and counts in
+// on the tile's counter, and the last adds the partials in k order
+// (deterministic) and runs the epilogue: the ticket pattern of
+// tfd::wait_stores_landed.  gridDim.y > 1 is the plain K split instead
+// (partial planes, then splitk_reduce_kernel), for so few tiles that one
+// workgroup would add too many partials.
+//
+// MFMA-bound: 124 TF/s at 999 x 3072 x 1024-like shapes once the split's 14 us
+// are paid; 4096 x 4096 x 2048 137 TF/s on shared units (146 as whole tiles),
+// 4-byte loads 2.2 us a unit instead of 1.9.  The dispatch rule (f32_plan)
+// has the measured times on both sides.
 // ---------------------------------------------------------------------------
 constexpr int kF32DlThreads = 512;
-constexpr int kF32DlStages = 4;
-constexpr int kF32DlOp = BM * kF32K;                                     // floats of one operand block
-constexpr int kF32DlLoads = kF32DlOp * 4 / 1024 / (kF32DlThreads / 64);  // 1 KB loads per wave per block
+enum F32Mode { kF32Whole, kF32Tail, kF32Words };
 
 __device__ __forceinline__ int f32dl_swz(int row) { return (row >> 1) & 7; }
 
+// Loads a wave issues per operand block of ROWS rows, and the bytes of each.
+constexpr int f32dl_load_bytes(int mode) { return mode == kF32Words ? 256 : 1024; }
+constexpr int f32dl_loads(int rows, int mode) { return rows * kF32K * 4 / f32dl_load_bytes(mode) / 8; }
+
 // Byte offsets (from the tile origin) of this lane's direct loads of one
-// operand block; wave w fills 1 KB pieces kF32DlLoads*w .. of it.
-template <bool KMAJ>
-__device__ __forceinline__ void f32dl_offsets(int64_t ld, uint32_t (&voff)[kF32DlLoads]) {
+// operand block, and each load's first k; wave w fills pieces L*w .. of it.
+template <bool KMAJ, int ROWS, int MODE, int L>
+__device__ __forceinline__ void f32dl_offsets(int64_t ld, uint32_t (&voff)[L], int (&kl)[L]) {
     const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
 #pragma unroll
-    for (int i = 0; i < kF32DlLoads; ++i) {
-        const int blk = w * kF32DlLoads + i;
+    for (int i = 0; i < L; ++i) {
+        const int blk = w * L + i;
+        int row, k;
         if (KMAJ) {
-            const int row = blk * 8 + (l >> 3);  // lane l fills slot l & 7 of row
-            voff[i] = 4u * ((uint32_t)row * (uint32_t)ld + 4u * (uint32_t)((l & 7) ^ f32dl_swz(row)));
+            // Lane l fills slot (l's) of a row; 4-byte loads one value of it.
+            row = MODE == kF32Words ? blk * 2 + (l >> 5) : blk * 8 + (l >> 3);
+            const int slot = MODE == kF32Words ? (l & 31) >> 2 : l & 7;
+            k = 4 * (slot ^ f32dl_swz(row)) + (MODE == kF32Words ? l & 3 : 0);
+            voff[i] = 4u * ((uint32_t)row * (uint32_t)ld + (uint32_t)k);
         } else {
-            const int k = blk * 2 + (l >> 5);
-            voff[i] = 4u * ((uint32_t)k * (uint32_t)ld + 4u * (uint32_t)(l & 31));
+            constexpr int lanes = MODE == kF32Words ? ROWS : ROWS / 4;   // lanes a k row
+            const int idx = blk * 64 + l;
+            k = idx / lanes;
+            row = (idx % lanes) * (MODE == kF32Words ? 1 : 4);
+            voff[i] = 4u * ((uint32_t)k * (uint32_t)ld + (uint32_t)row);
         }
+        kl[i] = k;
     }
 }
 
-// Issue this wave's direct loads of one operand block (M0 = the 1 KB LDS
-// destination; inline assembly for the reasons given at dl_issue).
-// `lds_wave`: LDS byte address of this wave's first 1 KB of the block.
-__device__ __forceinline__ void f32dl_issue(i32x4 rsrc, uint32_t tile_off, const uint32_t (&voff)[kF32DlLoads],
-                                            uint32_t lds_wave) {
-    static_for<kF32DlLoads>([&](auto I) TF_LAMBDA_INLINE {
-        constexpr int i = decltype(I)::value;
-        const uint32_t dst = lds_wave + i * 1024u;
-        const uint32_t v = voff[i], so = tile_off;  // asm operands must be locals of the lambda
-        const i32x4 r = rsrc;
+// One direct load (M0 = its LDS destination; inline assembly for the reasons
+// given at dl_issue).
+template <int MODE>
+__device__ __forceinline__ void f32dl_load(i32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t dst) {
+    if constexpr (MODE == kF32Words)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                     :
+                     : "s"(dst), "v"(voff), "s"(rsrc), "s"(soff)
+                     : "memory", "m0");
+    else
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                      :
-                     : "s"(dst), "v"(v), "s"(r), "s"(so)
+                     : "s"(dst), "v"(voff), "s"(rsrc), "s"(soff)
                      : "memory", "m0");
-    });
 }
 
 // One quad's fragments of one operand: the value of sub-tile i at step s.
-template <bool KMAJ>
+template <bool KMAJ, int NSUB>
 struct F32DlFrag;
-template <>
-struct F32DlFrag<true> {
-    f32x4 v[2];
+template <int NSUB>
+struct F32DlFrag<true, NSUB> {
+    f32x4 v[NSUB];
     __device__ __forceinline__ float at(int i, int s) const { return v[i][s]; }
 };
 template <>
-struct F32DlFrag<false> {
+struct F32DlFrag<false, 2> {
     f32x2 v[4];
     __device__ __forceinline__ float at(int i, int s) const { return v[s][i]; }
 };
+template <>
+struct F32DlFrag<false, 1> {
+    float v[4];
+    __device__ __forceinline__ float at(int, int s) const { return v[s]; }
+};
 
 // Per-lane LDS word offsets of one operand's fragment reads (wave rows
-// wbase .. wbase + 63, quads 2g + qq).  K-major: sub-tile i's row for quad
-// qq (swizzled chunk 4h + 2g + qq).  MN-major: the lane's row pair in k row
-// 16h + 8g.
-template <bool KMAJ>
+// wbase .. wbase + 32 NSUB - 1, quads 2g + qq).  K-major: sub-tile i's row for
+// quad qq (swizzled chunk 4h + 2g + qq).  MN-major: the lane's row (pair) in
+// k row 16h + 8g.
+template <bool KMAJ, int NSUB>
 struct F32DlOperand {
-    int off[KMAJ ? 4 : 1];
+    static constexpr int kRows = 64 * NSUB;
+    static constexpr int kReads = KMAJ ? NSUB : 4;   // LDS reads per quad
+    int off[KMAJ ? 2 * NSUB : 1];
     __device__ __forceinline__ void init(int wbase, int g) {
         const int l = threadIdx.x & 63, h = l >> 5, l32 = l & 31;
         if constexpr (KMAJ) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
+            for (int i = 0; i < NSUB; ++i) {
                 const int r = wbase + 32 * i + l32;
 #pragma unroll
                 for (int qq = 0; qq < 2; ++qq)
                     off[2 * i + qq] = r * kF32K + 4 * ((4 * h + 2 * g + qq) ^ f32dl_swz(r));
             }
         } else {
-            off[0] = (16 * h + 8 * g) * BM + wbase + 2 * l32;
+            off[0] = (16 * h + 8 * g) * kRows + wbase + NSUB * l32;
         }
     }
-    __device__ __forceinline__ void read(const float* op, int qq, F32DlFrag<KMAJ>& d) const {
+    __device__ __forceinline__ void read(const float* op, int qq, F32DlFrag<KMAJ, NSUB>& d) const {
         if constexpr (KMAJ) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i) d.v[i] = *reinterpret_cast<const f32x4*>(op + off[2 * i + qq]);
+            for (int i = 0; i < NSUB; ++i) d.v[i] = *reinterpret_cast<const f32x4*>(op + off[2 * i + qq]);
         } else {
 #pragma unroll
-            for (int s = 0; s < 4; ++s) d.v[s] = *reinterpret_cast<const f32x2*>(op + off[0] + (4 * qq + s) * BM);
+            for (int s = 0; s < 4; ++s) {
+                const float* src = op + off[0] + (4 * qq + s) * kRows;
+                if constexpr (NSUB == 2) d.v[s] = *reinterpret_cast<const f32x2*>(src);
+                else d.v[s] = *src;
+            }
         }
     }
 };
 
-constexpr int kF32DlPairFloats = 8 * 8 * 64 * 4;  // LDS floats of the pair reduction (8 KB per wave)
+// The even split of a product's units over workgroups (see the work split
+// above): the first `rem` of them take per + 1.
+__device__ __forceinline__ int unit_start(int w, int per, int rem) { return w * per + min(w, rem); }
+__device__ __forceinline__ int unit_owner(int u, int per, int rem) {
+    const int head = rem * (per + 1);
+    return u < head ? u / (per + 1) : rem + (u - head) / per;
+}
+
+// Values a wave keeps of its 32 MI x 32 NI block after the pair reduction.
+template <int MI, int NI>
+constexpr int kKeep = 8 * MI * NI;
 
 // Pair reduction through LDS of waves w and w ^ 4, which hold two k halves of
-// one 64 x 64 block: wave w hands sub-tile row block 1 - g to its partner and
-// keeps block g, complete (8 KB per wave, 1 KB per vector).  The caller has
-// synchronised the workgroup.
-__device__ __forceinline__ void pair_reduce(v16f (&acc)[2][2], int g, float* __restrict__ lds) {
+// one block: wave w hands half of it to its partner and keeps the other,
+// complete.  Group g keeps sub-tile row block g (MI = 2; keep[16 j + r]) or
+// rows 16 g .. 16 g + 15 (MI = 1; keep[8 j + r % 8]).  The halves are chosen
+// by value: indexing acc with the run-time g (even under a branch per
+// candidate) made the compiler keep all accumulators in scratch memory.  The
+// caller has synchronised the workgroup.
+template <int MI, int NI>
+__device__ __forceinline__ void pair_reduce(const v16f (&acc)[MI][NI], int g, float* __restrict__ lds,
+                                            float (&keep)[kKeep<MI, NI>]) {
+    constexpr int KV = kKeep<MI, NI>, RJ = 8 * MI;   // values, values per j
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     f32x4* x = reinterpret_cast<f32x4*>(lds);
-    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
-        constexpr int i = decltype(I)::value;
-        if (i == g) return;
-        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
-            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
-            x[(wave * 8 + v) * 64 + lane] = f32x4{acc[i][j][r], acc[i][j][r + 1], acc[i][j][r + 2], acc[i][j][r + 3]};
+    static_for<KV / 4>([&](auto V) TF_LAMBDA_INLINE {
+        f32x4 give;
+        static_for<4>([&](auto E) TF_LAMBDA_INLINE {
+            constexpr int e = decltype(E)::value, i = 4 * decltype(V)::value + e, j = i / RJ, r = i % RJ;
+            const float v0 = acc[0][j][r], v1 = MI == 2 ? acc[MI - 1][j][r] : acc[0][j][(r + 8) % 16];
+            give[e] = g ? v0 : v1;
+            keep[i] = g ? v1 : v0;
         });
+        x[(wave * (KV / 4) + decltype(V)::value) * 64 + lane] = give;
     });
     __syncthreads();
-    static_for<2>([&](auto I) TF_LAMBDA_INLINE {
-        constexpr int i = decltype(I)::value;
-        if (i != g) return;
-        static_for<8>([&](auto V) TF_LAMBDA_INLINE {
-            constexpr int v = decltype(V)::value, j = v >> 2, r = 4 * (v & 3);
-            const f32x4 y = x[((wave ^ 4) * 8 + v) * 64 + lane];
-            acc[i][j][r] += y[0];
-            acc[i][j][r + 1] += y[1];
-            acc[i][j][r + 2] += y[2];
-            acc[i][j][r + 3] += y[3];
-        });
+    static_for<KV / 4>([&](auto V) TF_LAMBDA_INLINE {
+        constexpr int v = decltype(V)::value;
+        const f32x4 y = x[((wave ^ 4) * (KV / 4) + v) * 64 + lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) keep[4 * v + e] += y[e];
     });
 }
 
-// Epilogue of the direct fp32 kernel for interior blocks without beta * C or
-// a row bias.  The wave's 32 x 64 block (sub-tile row block g after the pair
-// reduction) is staged in its own 8 KB of LDS (`stage`, 32 rows x 64
-// floats) and written by whole rows: a lane takes 4 consecutive columns
-// (16-byte stores; 16 lanes per row, 4 rows per pass), the pointer advances
-// by 4 staged rows per pass, and the output form (OUT 0: split-K partial,
-// 1: bf16, 2: fp32) and transform (XF 0: copy, 1: alpha * v + bias, 2: the
-// same then ReLU) are fixed at compile time.  Writing element by element
-// (store_wave) spends more time on address arithmetic and checks than on the
-// stores.  Staged row rl of block g is row rl (A_PAIR: 2 rl + g; otherwise
-// 32 g + rl) of the wave block; its column c is column c of the wave block
-// (B_PAIR: accumulator j holds columns 2 l + j, so a lane's pair of
-// accumulators is one 8-byte LDS write).  Returns false, having written
-// nothing, when the block does not qualify.
-template <bool A_PAIR, bool B_PAIR>
-__device__ __forceinline__ bool f32dl_store_fast(const GemmParams& p, const v16f (&acc)[2][2], int g, int m_base,
-                                                 int n_base, int64_t boff, int split, float* __restrict__ stage) {
+// LDS floats of the pair reduction and of the epilogue's staging (both per
+// workgroup of eight waves).
+template <int MI, int NI>
+constexpr int kPairFloats = 8 * kKeep<MI, NI> * 64;
+
+// Epilogue of a wave's kept half block.  It is staged in the wave's own part
+// of LDS (`stage`, 16 MI rows x 32 NI floats) and written by whole rows.
+// Without beta * C or a row bias: 16-byte stores where C allows them, else a
+// value a lane, the pointer advancing by whole passes, the output form (OUT
+// 0: a fp32 plane of leading dimension N, 1: bf16, 2: fp32) and transform (XF
+// 0: copy, 1: alpha * v + bias, 2: the same then ReLU) fixed at compile time,
+// rows past M skipped.  Writing element by element from the accumulators spends
+// more time on address arithmetic and checks than on the stores.
+// Staged row rl is row 16 g + rl of the block (MI = 1), 2 rl + g (A_PAIR) or
+// 32 g + rl; its column c is column c of the block (B_PAIR: accumulator j
+// holds columns 2 l + j, so a lane's pair is one 8-byte LDS write).
+// `plane`: write raw values there instead of C.
+template <int MI, int NI, bool A_PAIR, bool B_PAIR>
+__device__ __forceinline__ void tile_store(const GemmParams& p, const float (&keep)[kKeep<MI, NI>], int g, int m_base,
+                                           int n_base, int64_t boff, float* __restrict__ plane,
+                                           float* __restrict__ stage) {
+    constexpr int RJ = 8 * MI, ROWS = 16 * MI, W = 32 * NI;
+    constexpr int LPR = W / 4, RPP = 64 / LPR, PASSES = ROWS / RPP;   // vector copy: lanes a row, rows a pass
     const bool has_bias = p.epi != TF_EPI_NONE && p.epi != TF_EPI_RELU;
     const bool relu = p.epi == TF_EPI_BIAS_RELU || p.epi == TF_EPI_RELU || p.epi == TF_EPI_ROW_BIAS_RELU;
-    float* part = p.partial ? p.partial + (int64_t)split * p.M * p.N : nullptr;
-    if (!part && (p.beta != 0.0f || (has_bias && p.row_bias))) return false;
-    if (part ? p.N % 4 != 0 : p.vec_c4 == 0) return false;
-    if (m_base + 64 > p.M || n_base + 64 > p.N) return false;
     const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
-    // The kept block, chosen by value: indexing acc with the run-time g
-    // (even under a branch per candidate) made the compiler keep all
-    // accumulators in scratch memory.
-    const v16f k0 = g ? acc[1][0] : acc[0][0];
-    const v16f k1 = g ? acc[1][1] : acc[0][1];
-    static_for<16>([&](auto R) TF_LAMBDA_INLINE {
+    static_for<RJ>([&](auto R) TF_LAMBDA_INLINE {
         constexpr int r = decltype(R)::value;
-        float* row = stage + (8 * (r >> 2) + 4 * half + (r & 3)) * 64;
-        if constexpr (B_PAIR) {
-            *reinterpret_cast<f32x2*>(row + 2 * l32) = f32x2{k0[r], k1[r]};
+        float* row = stage + (8 * (r >> 2) + 4 * half + (r & 3)) * W;
+        if constexpr (NI == 2 && B_PAIR) {
+            *reinterpret_cast<f32x2*>(row + 2 * l32) = f32x2{keep[r], keep[RJ + r]};
         } else {
-            row[l32] = k0[r];
-            row[32 + l32] = k1[r];
+            static_for<NI>([&](auto J) TF_LAMBDA_INLINE { row[32 * J + l32] = keep[RJ * J + r]; });
         }
     });
-    const int rsub = lane >> 4, c4 = 4 * (lane & 15);
-    const int col = n_base + c4;
-    float cb[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) cb[e] = has_bias ? p.bias[col + e] : 0.0f;
+    constexpr int row_mul = MI == 2 && A_PAIR ? 2 : 1;   // rows of C per staged row
+    const int row_base = m_base + (MI == 1 ? 16 * g : A_PAIR ? g : 32 * g);
     const float alpha = p.alpha;
-    const int row_step = A_PAIR ? 2 : 1;  // rows of C per staged row
-    const int row0 = m_base + (A_PAIR ? g : 32 * g) + row_step * rsub;
-    const float* src = stage + rsub * 64 + c4;
-    auto copy = [&](auto OUT, auto XF) TF_LAMBDA_INLINE {
-        constexpr int out = decltype(OUT)::value, xf = decltype(XF)::value;
-        using Dst = std::conditional_t<out == 1, uint16_t, float>;
-        const int64_t ld = out == 0 ? (int64_t)p.N : (int64_t)p.ldc;
-        Dst* dst = out == 0 ? reinterpret_cast<Dst*>(part) + (int64_t)row0 * ld + col
-                            : reinterpret_cast<Dst*>(p.C) + boff + (int64_t)row0 * ld + col;
-#pragma unroll
-        for (int pass = 0; pass < 8; ++pass) {
-            f32x4 o = *reinterpret_cast<const f32x4*>(src + pass * 4 * 64);
-            if constexpr (xf != 0) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float t = alpha * o[e] + cb[e];
-                    o[e] = xf == 2 ? fmaxf(t, 0.0f) : t;
-                }
-            }
-            if constexpr (out == 1)
-                *reinterpret_cast<uint2*>(dst) = make_uint2(tfd::bf16x2_rne(o[0], o[1]), tfd::bf16x2_rne(o[2], o[3]));
-            else
-                *reinterpret_cast<f32x4*>(dst) = o;
-            dst += 4 * row_step * ld;
-        }
-    };
+    const bool loads = !plane && (p.beta != 0.0f || (has_bias && p.row_bias));
     using I0 = std::integral_constant<int, 0>;
     using I1 = std::integral_constant<int, 1>;
     using I2 = std::integral_constant<int, 2>;
+    // The output form and transform of a copy, chosen once.
     const bool plain = alpha == 1.0f && !has_bias && !relu;
-    if (part) copy(I0{}, I0{});
-    else if (p.out_bf16) {
-        if (plain) copy(I1{}, I0{});
-        else if (relu) copy(I1{}, I2{});
-        else copy(I1{}, I1{});
-    } else {
-        if (plain) copy(I2{}, I0{});
-        else if (relu) copy(I2{}, I2{});
-        else copy(I2{}, I1{});
+    auto with_form = [&](auto copy) TF_LAMBDA_INLINE {
+        if (plane) copy(I0{}, I0{});
+        else if (p.out_bf16) {
+            if (plain) copy(I1{}, I0{});
+            else if (relu) copy(I1{}, I2{});
+            else copy(I1{}, I1{});
+        } else {
+            if (plain) copy(I2{}, I0{});
+            else if (relu) copy(I2{}, I2{});
+            else copy(I2{}, I1{});
+        }
+    };
+    if (!loads && (plane ? p.N % 4 == 0 : p.vec_c4 != 0 && p.N % 4 == 0)) {
+        const int rsub = lane / LPR, c4 = 4 * (lane % LPR);
+        const int col = n_base + c4, row0 = row_base + row_mul * rsub;
+        if (col >= p.N) return;   // N % 4 == 0: a lane's columns are all inside or all outside
+        float cb[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) cb[e] = has_bias && !plane ? p.bias[col + e] : 0.0f;
+        const float* src = stage + rsub * W + c4;
+        // Rows of this lane's inside C: all of them in an interior block.
+        const int rows = min(PASSES, (p.M - row0 + RPP * row_mul - 1) / (RPP * row_mul));
+        with_form([&](auto OUT, auto XF) TF_LAMBDA_INLINE {
+            constexpr int out = decltype(OUT)::value, xf = decltype(XF)::value;
+            using Dst = std::conditional_t<out == 1, uint16_t, float>;
+            const int64_t ld = out == 0 ? (int64_t)p.N : (int64_t)p.ldc;
+            Dst* dst = out == 0 ? reinterpret_cast<Dst*>(plane) + (int64_t)row0 * ld + col
+                                : reinterpret_cast<Dst*>(p.C) + boff + (int64_t)row0 * ld + col;
+#pragma unroll
+            for (int pass = 0; pass < PASSES; ++pass) {
+                f32x4 o = *reinterpret_cast<const f32x4*>(src + pass * RPP * W);
+                if constexpr (xf != 0) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float t = alpha * o[e] + cb[e];
+                        o[e] = xf == 2 ? fmaxf(t, 0.0f) : t;
+                    }
+                }
+                if (pass < rows) {
+                    if constexpr (out == 1)
+                        *reinterpret_cast<uint2*>(dst) =
+                            make_uint2(tfd::bf16x2_rne(o[0], o[1]), tfd::bf16x2_rne(o[2], o[3]));
+                    else
+                        *reinterpret_cast<f32x4*>(dst) = o;
+                }
+                dst += RPP * row_mul * ld;
+            }
+        });
+        return;
     }
+    // A value a lane.
+    constexpr int SRPP = 64 / W, SPASSES = ROWS / SRPP;   // rows a pass (W lanes each)
+    const int rsub = lane / W, c = lane % W, col = n_base + c, row0 = row_base + row_mul * rsub;
+    if (col >= p.N) return;
+    const float cb = has_bias && !p.row_bias && !plane ? p.bias[col] : 0.0f;
+    const float* src = stage + rsub * W + c;
+    const int rows = min(SPASSES, (p.M - row0 + SRPP * row_mul - 1) / (SRPP * row_mul));
+    if (!loads) {
+        with_form([&](auto OUT, auto XF) TF_LAMBDA_INLINE {
+            constexpr int out = decltype(OUT)::value, xf = decltype(XF)::value;
+            using Dst = std::conditional_t<out == 1, uint16_t, float>;
+            const int64_t ld = out == 0 ? (int64_t)p.N : (int64_t)p.ldc;
+            Dst* dst = out == 0 ? reinterpret_cast<Dst*>(plane) + (int64_t)row0 * ld + col
+                                : reinterpret_cast<Dst*>(p.C) + boff + (int64_t)row0 * ld + col;
+#pragma unroll 8
+            for (int pass = 0; pass < SPASSES; ++pass) {
+                float v = src[pass * SRPP * W];
+                if constexpr (xf != 0) v = alpha * v + cb;
+                if constexpr (xf == 2) v = fmaxf(v, 0.0f);
+                if (pass < rows) {
+                    if constexpr (out == 1) *dst = tfd::f32_to_bf16(v);
+                    else *dst = v;
+                }
+                dst += SRPP * row_mul * ld;
+            }
+        });
+        return;
+    }
+    // beta * C or a row bias: loads among the stores (this GPU counts both in
+    // one counter, so waiting for a load waits for every store before it).
+    for (int pass = 0; pass < rows; ++pass) {
+        const int row = row0 + SRPP * row_mul * pass;
+        const int64_t off = boff + (int64_t)row * p.ldc + col;
+        const float rb = has_bias && p.row_bias ? p.bias[row] : 0.0f;
+        emit(p, off, src[pass * SRPP * W], cb + rb, relu);
+    }
+}
+
+// Adds the partial tiles of the workgroups that share tile `tile` (units
+// [tile * kblk, (tile + 1) * kblk)); true in the last one to arrive, whose
+// `keep` then holds the sum.  Workgroup w stores its share in slot 2 w + 1
+// (its last segment, which begins the tile) or 2 w (its first, which does
+// not).  Every thread of the workgroup calls it.
+template <int KV>
+__device__ __forceinline__ bool combine_shares(const GemmParams& p, int tile, int w, float (&keep)[KV]) {
+    const int first = unit_owner(tile * p.units_tile, p.units_per, p.units_rem);
+    const int n = unit_owner(tile * p.units_tile + p.units_tile - 1, p.units_per, p.units_rem) - first + 1;
+    if (n == 1) return true;
+    __shared__ bool last;
+    const int64_t slot_floats = (int64_t)KV * 512;
+    float* mine = p.partial + (2 * w + (w == first ? 1 : 0)) * slot_floats + threadIdx.x;
+#pragma unroll
+    for (int v = 0; v < KV; ++v)
+        __hip_atomic_store(mine + v * 512, keep[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    tfd::wait_stores_landed();
+    __syncthreads();
+    if (threadIdx.x == 0)
+        last = __hip_atomic_fetch_add(p.tickets + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ==
+               (unsigned)(n - 1);
+    __syncthreads();
+    if (!last) return false;
+    float own[KV];
+#pragma unroll
+    for (int v = 0; v < KV; ++v) own[v] = keep[v];
+    for (int c = 0; c < n; ++c) {
+        const float* src = p.partial + (2 * (first + c) + (c == 0 ? 1 : 0)) * slot_floats + threadIdx.x;
+        float t[KV];
+        if (first + c == w) {
+#pragma unroll
+            for (int v = 0; v < KV; ++v) t[v] = own[v];
+        } else {
+#pragma unroll
+            for (int v = 0; v < KV; ++v)
+                t[v] = __hip_atomic_load(src + v * 512, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int v = 0; v < KV; ++v) keep[v] = c == 0 ? t[v] : keep[v] + t[v];
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(p.tickets + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
 }
 
+// Workgroup number with the numbers one XCD receives (id % 8) made contiguous.
+__device__ __forceinline__ int xcd_contiguous(int wg, int total) {
+    return (total & 7) == 0 ? (wg & 7) * (total >> 3) + (wg >> 3) : wg;
+}
+
+// 64-wide tiles: a ring of three blocks (72 KB) and at most 128 registers, so
+// two workgroups share a CU; 128 x 128: a ring of four (128 KB).
+template <int MI, int NI>
+constexpr int kF32DlStages = MI + NI == 4 ? 4 : 3;
+
+// SHARED: the even split of units (gridDim.y == 1).  Otherwise workgroup
+// (w, split) takes a k range of tile w (all of it with gridDim.y == 1): the
+// same code without the segment loop and its scalars.
+template <bool A_KMAJ, bool B_KMAJ, int MI, int NI, int MODE, bool SHARED>
+__global__ __launch_bounds__(kF32DlThreads, MI + NI == 4 ? 2 : 4) void gemm_f32_dl_kernel(GemmParams p) {
+    constexpr int S = kF32DlStages<MI, NI>;
+    constexpr int kOpA = 64 * MI * kF32K, kOpB = 64 * NI * kF32K, kStage = kOpA + kOpB;   // floats
+    constexpr int LA = f32dl_loads(64 * MI, MODE), LB = f32dl_loads(64 * NI, MODE), kPiece = f32dl_load_bytes(MODE);
+    __shared__ __attribute__((aligned(16))) float lds[S * kStage];
+    const int w = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int split = blockIdx.y;
+    const int wave = threadIdx.x >> 6;
+    const int g = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    const int kpb = (p.K + kF32K - 1) / kF32K;
+
+    F32DlOperand<A_KMAJ, MI> oa;
+    F32DlOperand<B_KMAJ, NI> ob;
+    oa.init(wm * 32 * MI, g);
+    ob.init(wn * 32 * NI, g);
+    uint32_t voff_a[LA], voff_b[LB];
+    int kl_a[LA], kl_b[LB];
+    f32dl_offsets<A_KMAJ, 64 * MI, MODE>(p.lda, voff_a, kl_a);
+    f32dl_offsets<B_KMAJ, 64 * NI, MODE>(p.ldb, voff_b, kl_b);
+    const uint32_t a_kstep = 4u * kF32K * (A_KMAJ ? 1u : (uint32_t)p.lda);
+    const uint32_t b_kstep = 4u * kF32K * (B_KMAJ ? 1u : (uint32_t)p.ldb);
+    const uint32_t lds_a = lds_addr(lds) + (uint32_t)__builtin_amdgcn_readfirstlane(wave * LA * kPiece);
+    const uint32_t lds_b = lds_addr(lds) + kOpA * 4 + (uint32_t)__builtin_amdgcn_readfirstlane(wave * LB * kPiece);
+
+    int u = SHARED ? unit_start(w, p.units_per, p.units_rem) : 0;
+    const int u_end = SHARED ? unit_start(w + 1, p.units_per, p.units_rem) : 0;
+    do {
+        const int tile = SHARED ? u / p.units_tile : w;
+        const int kb_beg = SHARED ? u - tile * p.units_tile : split * p.kb_per_split;
+        const int nk = min(p.units_tile, kb_beg + (SHARED ? u_end - u : p.kb_per_split)) - kb_beg;
+        u += nk;
+        const int per_batch = p.tiles_m * p.tiles_n;
+        const int batch = tile / per_batch;
+        int tm, tn;
+        grouped_tile(tile - batch * per_batch, p.tiles_m, p.tiles_n, tm, tn);
+        const int m0 = tm * 64 * MI, n0 = tn * 64 * NI;
+        const float* A = reinterpret_cast<const float*>(p.A) + (int64_t)batch * p.stride_a;
+        const float* B = reinterpret_cast<const float*>(p.B) + (int64_t)batch * p.stride_b;
+        v16f acc[MI][NI];
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) acc[i][j] = v16f{};
+        struct Quad {
+            F32DlFrag<A_KMAJ, MI> a;
+            F32DlFrag<B_KMAJ, NI> b;
+        };
+        Quad f[2];
+        auto stage_a = [&](int st) TF_LAMBDA_INLINE { return lds + st * kStage; };
+        KWalk walk;
+        walk.init(A, B, 4 * p.stride_a, 4 * p.stride_b, kb_beg, nk, kpb);
+        const uint32_t ta0 = 4u * (A_KMAJ ? (uint32_t)m0 * (uint32_t)p.lda : (uint32_t)m0);
+        const uint32_t tb0 = 4u * (B_KMAJ ? (uint32_t)n0 * (uint32_t)p.ldb : (uint32_t)n0);
+        // The walk's next block: descriptors, scalar offsets, the k it holds.
+        struct Next {
+            i32x4 ra, rb;
+            uint32_t so_a, so_b;
+            int rem;
+        };
+        auto next_block = [&]() TF_LAMBDA_INLINE {
+            const Next n{dl_rsrc(walk.a_base, p.a_bytes), dl_rsrc(walk.b_base, p.b_bytes),
+                         ta0 + (uint32_t)walk.kin * a_kstep, tb0 + (uint32_t)walk.kin * b_kstep,
+                         p.K - walk.kin * kF32K};
+            walk.advance();
+            return n;
+        };
+        Next n = next_block();
+        // Load x of its LA + LB into stage st.
+        auto issue = [&](const Next& n, int st, auto X) TF_LAMBDA_INLINE {
+            constexpr int x = decltype(X)::value;
+            const uint32_t dst = (uint32_t)(st * kStage * 4);
+            if constexpr (x < LA) {
+                const uint32_t v = kl_a[x] < n.rem ? voff_a[x] : kDlOob;
+                f32dl_load<MODE>(n.ra, v, n.so_a, lds_a + dst + x * kPiece);
+            } else {
+                constexpr int y = x - LA;
+                const uint32_t v = kl_b[y] < n.rem ? voff_b[y] : kDlOob;
+                f32dl_load<MODE>(n.rb, v, n.so_b, lds_b + dst + y * kPiece);
+            }
+        };
+        auto read = [&](int st, int qq, Quad& d) TF_LAMBDA_INLINE {
+            oa.read(stage_a(st), qq, d.a);
+            ob.read(stage_a(st) + kOpA, qq, d.b);
+        };
+        constexpr int NM = 4 * MI * NI;   // MFMAs of a quad
+        auto mfma = [&](const Quad& d, auto Mc) TF_LAMBDA_INLINE {
+            constexpr int m = decltype(Mc)::value, s = m / (MI * NI), i = m / NI % MI, j = m % NI;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(d.a.at(i, s), d.b.at(j, s), acc[i][j], 0, 0, 0);
+        };
+        auto mfma_quad = [&](const Quad& d) TF_LAMBDA_INLINE {
+            static_for<NM>([&](auto Mc) TF_LAMBDA_INLINE { mfma(d, Mc); });
+        };
+        constexpr int kRd = F32DlOperand<A_KMAJ, MI>::kReads + F32DlOperand<B_KMAJ, NI>::kReads;
+        auto pin_reads = [&]() TF_LAMBDA_INLINE {
+            static_for<kRd>([&](auto) TF_LAMBDA_INLINE {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // DS read
+            });
+        };
+        // Block t in stage b = t % S (this wave's two quads of it).  Every
+        // block but the last waits for block t+1 (S-3 newer blocks of loads
+        // stay in flight), which also guarantees every wave is done with block
+        // t-1's stage, loads block t+S-1 (clamped to the last block: loads
+        // past the end land in stages nobody reads again) into that stage and
+        // reads block t+1's first fragments.  LAST: no next block.
+        auto block = [&](auto Bc, int t, auto LAST) TF_LAMBDA_INLINE {
+            constexpr int b = decltype(Bc)::value;
+            constexpr bool last = decltype(LAST)::value;
+            read(b, 1, f[1]);
+            mfma_quad(f[0]);
+            pin_reads();
+            __builtin_amdgcn_sched_barrier(0);
+            if constexpr (!last) {
+                dl_barrier<(S - 3) * (LA + LB)>();
+                // An MFMA first and between the loads (a wave whose load waits
+                // to issue would leave its matrix core idle), and the scalar
+                // work of the block after (n) between MFMAs too: ahead of the
+                // barrier it delayed every wave by its 110 cycles, 2.4 % of
+                // the k loop.
+                mfma(f[1], std::integral_constant<int, 0>{});
+                __builtin_amdgcn_sched_barrier(0);
+                read((b + 1) % S, 0, f[0]);
+                static_for<NM - 1>([&](auto Mc) TF_LAMBDA_INLINE {
+                    constexpr int m = decltype(Mc)::value + 1;
+                    constexpr int per = LA + LB <= 4 ? LA + LB : (LA + LB + NM - 2) / (NM - 1);
+                    mfma(f[1], std::integral_constant<int, m>{});
+                    static_for<per>([&](auto Y) TF_LAMBDA_INLINE {
+                        constexpr int x = (m - 1) * per + decltype(Y)::value;
+                        if constexpr (x < LA + LB)   // of block min(t + S - 1, nk - 1)
+                            issue(n, (b + S - 1) % S, std::integral_constant<int, x>{});
+                        if constexpr (x == LA + LB - 1) n = next_block();
+                    });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            } else {
+                mfma_quad(f[1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        // Prologue: blocks 0 .. S-2 (clamped) into stages 0 .. S-2, wait for block 0.
+        static_for<S - 1>([&](auto Bc) TF_LAMBDA_INLINE {
+            constexpr int b = decltype(Bc)::value;
+            static_for<LA + LB>([&](auto X) TF_LAMBDA_INLINE { issue(n, b, X); });
+            n = next_block();  // block min(b + 1, nk - 1)
+        });
+        dl_barrier<(S - 2) * (LA + LB)>();
+        read(0, 0, f[0]);
+        // Blocks 0 .. nk-2, S per iteration (stage = position in the group)
+        // and what is left of them.  (One loop with an exit test per block
+        // was compiled into two loops: 2 % slower at 2048 x 2048 x 2048.)
+        int t = 0;
+        for (; t + S < nk; t += S)
+            static_for<S>([&](auto Bc) TF_LAMBDA_INLINE { block(Bc, t + decltype(Bc)::value, std::false_type{}); });
+        static_for<S - 1>([&](auto Bc) TF_LAMBDA_INLINE {
+            if (t + 1 < nk) {
+                block(Bc, t, std::false_type{});
+                ++t;
+            }
+        });
+        // Block nk-1.
+        const int rlast = t % S;
+        static_for<S>([&](auto Bc) TF_LAMBDA_INLINE {
+            if (rlast == decltype(Bc)::value) block(Bc, t, std::true_type{});
+        });
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the clamped loads
+        __syncthreads();  // every wave is done with the stages
+        float keep[kKeep<MI, NI>];
+        pair_reduce<MI, NI>(acc, g, lds, keep);
+        const int mb = m0 + wm * 32 * MI, nb = n0 + wn * 32 * NI;
+        float* stage = lds + kPairFloats<MI, NI> + wave * kKeep<MI, NI> * 64;
+        static_assert(2 * kPairFloats<MI, NI> <= S * kStage, "pair reduction and staging must fit in the ring");
+        if constexpr (SHARED) {
+            if (combine_shares<kKeep<MI, NI>>(p, tile, w, keep))
+                tile_store<MI, NI, !A_KMAJ, !B_KMAJ>(p, keep, g, mb, nb, (int64_t)batch * p.stride_c, nullptr, stage);
+            __syncthreads();  // the next segment's loads reuse the ring
+        } else {
+            float* plane = p.partial ? p.partial + (int64_t)split * p.M * p.N : nullptr;
+            tile_store<MI, NI, !A_KMAJ, !B_KMAJ>(p, keep, g, mb, nb, (int64_t)batch * p.stride_c, plane, stage);
+        }
+    } while (SHARED && u < u_end);
+}
+
+// The 128 x 128 tile in one piece, 16-byte loads, K % 32 == 0: products whose
+// tiles come in whole rounds.  The same tile, ring and k order as
+// gemm_f32_dl_kernel (so the same bits); its k loop, without the segments and
+// the masks, is 2.5 % faster where B is MN-major (2048 x 2048 x 4096: 233.5
+// us against 239.5) and alike where it is K-major (239.5).
 template <bool A_KMAJ, bool B_KMAJ>
-__global__ __launch_bounds__(kF32DlThreads) void gemm_f32_dl_kernel(GemmParams p) {
-    constexpr int S = kF32DlStages;
+__global__ __launch_bounds__(kF32DlThreads) void gemm_f32_whole_kernel(GemmParams p) {
+    constexpr int S = 4, kF32DlOp = BM * kF32K, kF32DlLoads = f32dl_loads(BM, kF32Whole);
     __shared__ __attribute__((aligned(16))) float lds[S * 2 * kF32DlOp];
     int tm, tn;
     tile_coords(blockIdx.x, p.tiles_m, p.tiles_n, tm, tn);
@@ -2089,16 +2449,17 @@ __global__ __launch_bounds__(kF32DlThreads) void gemm_f32_dl_kernel(GemmParams p
         for (int j = 0; j < 2; ++j) acc[i][j] = v16f{};
 
     if (nk > 0) {
-        F32DlOperand<A_KMAJ> oa;
-        F32DlOperand<B_KMAJ> ob;
+        F32DlOperand<A_KMAJ, 2> oa;
+        F32DlOperand<B_KMAJ, 2> ob;
         oa.init(wm * 64, g);
         ob.init(wn * 64, g);
         uint32_t voff_a[kF32DlLoads], voff_b[kF32DlLoads];
-        f32dl_offsets<A_KMAJ>(p.lda, voff_a);
-        f32dl_offsets<B_KMAJ>(p.ldb, voff_b);
+        int unused[kF32DlLoads];
+        f32dl_offsets<A_KMAJ, BM, kF32Whole>(p.lda, voff_a, unused);
+        f32dl_offsets<B_KMAJ, BM, kF32Whole>(p.ldb, voff_b, unused);
         struct Quad {
-            F32DlFrag<A_KMAJ> a;
-            F32DlFrag<B_KMAJ> b;
+            F32DlFrag<A_KMAJ, 2> a;
+            F32DlFrag<B_KMAJ, 2> b;
         };
         Quad f[2];
         auto stage_a = [&](int st) TF_LAMBDA_INLINE { return lds + st * 2 * kF32DlOp; };
@@ -2112,8 +2473,8 @@ __global__ __launch_bounds__(kF32DlThreads) void gemm_f32_dl_kernel(GemmParams p
         const uint32_t wave_lds = lds_addr(lds) + dl_wave_offset<kF32DlLoads>();
         auto issue_next = [&](int st) TF_LAMBDA_INLINE {
             const uint32_t dst = wave_lds + (uint32_t)(st * 2 * kF32DlOp * 4);
-            f32dl_issue(dl_rsrc(walk.a_base, p.a_bytes), ta0 + (uint32_t)walk.kin * a_kstep, voff_a, dst);
-            f32dl_issue(dl_rsrc(walk.b_base, p.b_bytes), tb0 + (uint32_t)walk.kin * b_kstep, voff_b,
+            dl_issue<kF32DlLoads>(dl_rsrc(walk.a_base, p.a_bytes), ta0 + (uint32_t)walk.kin * a_kstep, voff_a, dst);
+            dl_issue<kF32DlLoads>(dl_rsrc(walk.b_base, p.b_bytes), tb0 + (uint32_t)walk.kin * b_kstep, voff_b,
                         dst + kF32DlOp * 4);
             walk.advance();
         };
@@ -2189,12 +2550,10 @@ __global__ __launch_bounds__(kF32DlThreads) void gemm_f32_dl_kernel(GemmParams p
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));  // drain the clamped loads
     }
     __syncthreads();  // every wave is done with the stages
-    pair_reduce(acc, g, lds);
-    static_assert(kF32DlPairFloats + 8 * 32 * 64 <= S * 2 * kF32DlOp, "epilogue staging must fit in the ring");
-    float* stage = lds + kF32DlPairFloats + wave * 32 * 64;  // past the pair-reduction area
-    if (!f32dl_store_fast<!A_KMAJ, !B_KMAJ>(p, acc, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c,
-                                            split, stage))
-        store_wave<2, !A_KMAJ, !B_KMAJ>(p, acc, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split, g);
+    float keep[kKeep<2, 2>];
+    pair_reduce<2, 2>(acc, g, lds, keep);
+    tile_store<2, 2, !A_KMAJ, !B_KMAJ>(p, keep, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, nullptr,
+                                       lds + kPairFloats<2, 2> + wave * kKeep<2, 2> * 64);
 }
 
 // ---------------------------------------------------------------------------
@@ -2403,12 +2762,12 @@ void gemm_bf16_mid_kernel(GemmParams p) {
     }
     __syncthreads();  // every wave is done with the stages
     float* sf = reinterpret_cast<float*>(lds);
-    pair_reduce(acc, g, sf);
-    static_assert(kF32DlPairFloats + 8 * 32 * 64 <= S * 2 * kMidVec * 4, "epilogue staging must fit in the ring");
-    float* stage = sf + kF32DlPairFloats + wave * 32 * 64;
-    if (!f32dl_store_fast<false, false>(p, acc, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split,
-                                        stage))
-        store_wave<2, false, false>(p, acc, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, split, g);
+    float keep[kKeep<2, 2>];
+    pair_reduce<2, 2>(acc, g, sf, keep);
+    static_assert(2 * kPairFloats<2, 2> <= S * 2 * kMidVec * 4, "pair reduction and staging must fit in the ring");
+    float* plane = p.partial ? p.partial + (int64_t)split * p.M * p.N : nullptr;
+    tile_store<2, 2, false, false>(p, keep, g, m0 + wm * 64, n0 + wn * 64, (int64_t)batch * p.stride_c, plane,
+                                   sf + kPairFloats<2, 2> + wave * kKeep<2, 2> * 64);
 }
 
 // Small fp32 products (C1's layers, C4's fully connected layer): one block
@@ -2973,11 +3332,28 @@ KernelFn pick_bf16(bool a_kmaj, bool b_kmaj) {
     return gemm_bf16_kernel<BN, false, false>;
 }
 
+KernelFn pick_f32_whole(bool a_kmaj, bool b_kmaj) {
+    if (a_kmaj && b_kmaj) return gemm_f32_whole_kernel<true, true>;
+    if (a_kmaj && !b_kmaj) return gemm_f32_whole_kernel<true, false>;
+    if (!a_kmaj && b_kmaj) return gemm_f32_whole_kernel<false, true>;
+    return gemm_f32_whole_kernel<false, false>;
+}
+
+template <int MI, int NI, int MODE, bool SHARED>
 KernelFn pick_f32_dl(bool a_kmaj, bool b_kmaj) {
-    if (a_kmaj && b_kmaj) return gemm_f32_dl_kernel<true, true>;
-    if (a_kmaj && !b_kmaj) return gemm_f32_dl_kernel<true, false>;
-    if (!a_kmaj && b_kmaj) return gemm_f32_dl_kernel<false, true>;
-    return gemm_f32_dl_kernel<false, false>;
+    if (a_kmaj && b_kmaj) return gemm_f32_dl_kernel<true, true, MI, NI, MODE, SHARED>;
+    if (a_kmaj && !b_kmaj) return gemm_f32_dl_kernel<true, false, MI, NI, MODE, SHARED>;
+    if (!a_kmaj && b_kmaj) return gemm_f32_dl_kernel<false, true, MI, NI, MODE, SHARED>;
+    return gemm_f32_dl_kernel<false, false, MI, NI, MODE, SHARED>;
+}
+
+template <int MI, int NI>
+KernelFn pick_f32_dl(bool a_kmaj, bool b_kmaj, int mode, bool shared) {
+    if (mode == kF32Words)
+        return shared ? pick_f32_dl<MI, NI, kF32Words, true>(a_kmaj, b_kmaj)
+                      : pick_f32_dl<MI, NI, kF32Words, false>(a_kmaj, b_kmaj);
+    return shared ? pick_f32_dl<MI, NI, kF32Tail, true>(a_kmaj, b_kmaj)
+                  : pick_f32_dl<MI, NI, kF32Tail, false>(a_kmaj, b_kmaj);
 }
 
 KernelFn pick_bf16_big(bool a_kmaj, bool b_kmaj) {
@@ -3143,19 +3519,82 @@ Bf16Plan bf16_plan(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t batch, 
     return best;
 }
 
+// How the direct-to-LDS kernel runs an fp32 product: tile, and `groups`
+// workgroups that share its units evenly (0: one per tile and K slice) or
+// `splits` K slices.  Estimated in us from measured products (ncu = 256):
+//   128 x 128 whole tiles 10 + 1.71 a 32-deep block and round;
+//   shared units 14 + 1.9 a unit (2.2 with 4-byte loads), 4 more where the
+//   workgroups run over several tiles, and 0.5 per workgroup on a tile;
+//   K slices 15 + 1.9 a block, and 0.35 a MB of partials;
+//   the 64-wide tiles, two to a CU, take as long a unit as a 128 x 128 one
+//   does (half the work a unit at twice the units in flight), and 1.02 us
+//   alone on their CU.
+// Against the register-staged 128 x 64 kernel and its K split (us): 999 x 3072
+// x 1001 150-158 -> 70, 999 x 1001 x 3072 85-120 -> 58-68, 1000 x 3072 x 1024
+// 110-212 -> 60, 512 x 4096 x 2048 86-97 -> 69, 64 x 4096 x 4096 56-115 -> 35.
+struct F32Plan {
+    int MI, NI;
+    int64_t groups;
+    int splits;
+};
+F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t batch, int mode) {
+    F32Plan best{2, 2, 0, 1};
+    double least = 1e300;
+    const double unit = mode == kF32Words ? 2.2 : 1.9;
+    static const int shapes[3][2] = {{2, 2}, {2, 1}, {1, 2}};
+    for (const auto& s : shapes) {
+        const int64_t tiles = ((M + 64 * s[0] - 1) / (64 * s[0])) * ((N + 64 * s[1] - 1) / (64 * s[1])) * batch;
+        const bool wide = s[0] + s[1] == 4;
+        const int64_t slots = wide ? ncu : 2 * ncu, units = tiles * kblocks;
+        auto consider = [&](double t, int64_t groups, int splits) {
+            if (t < least) {
+                least = t;
+                best = F32Plan{s[0], s[1], groups, splits};
+            }
+        };
+        const double rounds = (double)((tiles + slots - 1) / slots);
+        if (wide) consider(rounds * (10.0 + (mode == kF32Whole ? 1.71 : unit) * (double)kblocks), 0, 1);
+        else if (tiles <= ncu) consider(8.0 + unit * 0.56 * (double)kblocks, 0, 1);
+        else consider(rounds * (8.0 + unit * (double)kblocks), 0, 1);
+        if (tiles <= tfh::kTicketGemmTiles && units >= 2 * slots && units < (int64_t(1) << 31) && tiles != slots)
+            consider(14.0 + unit * (double)((units + slots - 1) / slots) + (tiles > slots ? 4.0 : 0.0) +
+                         0.5 * (double)slots / (double)tiles, slots, 1);
+        const int64_t slices = std::min<int64_t>({slots / std::max<int64_t>(tiles, 1), kblocks / 4, 128});
+        if (batch == 1 && slices > 1)
+            consider(15.0 + unit * (double)((kblocks + slices - 1) / slices) +
+                         0.35 * (double)slices * (double)M * (double)N * 4e-6, 0, (int)slices);
+    }
+    return best;
+}
+
 // Grid of the small-product kernel for an M x N x K product: 32 x 32 tiles
 // and enough chunk groups for ~256 blocks, at most 32 per tile (the last
 // block adds them up), each of >= 1 chunk of 64 k.  False when the product
 // does not fit that kernel.
-bool small_grid(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t& tiles, int64_t& groups, int& cps) {
+// Longer K only in products of at most `long_limit` multiply-adds: 32 x 64 x
+// 4096 takes 14-21 us on the tile kernels with their K split.
+bool small_grid(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t& tiles, int64_t& groups, int& cps,
+                double long_limit = 0.0) {
     tiles = ((M + kSmT - 1) / kSmT) * ((N + kSmT - 1) / kSmT);
-    if (!(K > 0 && K <= 2048 && (double)M * (double)N * (double)K <= 134217728.0 && tiles <= tfh::kTicketGemmTiles))
+    const double work = (double)M * (double)N * (double)K;
+    if (!(K > 0 && (K <= 2048 ? work <= 134217728.0 : work <= long_limit) && tiles <= tfh::kTicketGemmTiles))
         return false;
     const int64_t nkc = (K + kSmKC - 1) / kSmKC;
     groups = std::min<int64_t>({nkc, 32, std::max<int64_t>(1, (ncu + tiles - 1) / tiles)});
     cps = (int)((nkc + groups - 1) / groups);
     groups = (nkc + cps - 1) / cps;
     return true;
+}
+
+// C = epi of the sum of p.partial's `splits` planes.
+tf_status launch_splitk_reduce(tf_ctx* ctx, const GemmParams& p, int splits) {
+    if (splits >= 16) {
+        splitk_reduce_wide_kernel<<<(unsigned)(((int64_t)p.M * p.N + 15) / 16), 256, 0, ctx->stream>>>(p, splits);
+    } else {
+        dim3 rgrid((unsigned)((p.N + 1023) / 1024), (unsigned)std::min(p.M, 65535));
+        splitk_reduce_kernel<<<rgrid, 256, 0, ctx->stream>>>(p, splits);
+    }
+    return tfh::check_launch("splitk_reduce_kernel");
 }
 
 // `noalloc`: split-K partials go to the fixed scratch array (no pool call).
@@ -3285,7 +3724,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     // gemm_f32_small_kernel).
     int64_t sm_tiles = 0, groups = 0;
     int cps = 0;
-    if (in_dtype == TF_F32 && batch == 1 && small_grid(ncu, M, N, K, sm_tiles, groups, cps)) {
+    if (in_dtype == TF_F32 && batch == 1 && small_grid(ncu, M, N, K, sm_tiles, groups, cps, mask_a ? 0.0 : 33554432.0)) {
         p.tiles_m = (int)((M + kSmT - 1) / kSmT);
         p.tiles_n = (int)((N + kSmT - 1) / kSmT);
         if (groups > 1) {
@@ -3334,23 +3773,45 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         p.int_n = direct ? (int)(part_n ? (N + kBigTile - 1) / kBigTile : N / kBigTile) : 0;
     }
 
-    // fp32 with 128 x 128 tiles: the tiles of an int_m x int_n grid take the
-    // direct-to-LDS kernel when K is a whole number of 32-deep blocks, the
-    // operands are 16-byte loadable and each extent fits the descriptor.
-    // Partial tiles at the M / N edges are fine for it as for the bf16 one;
-    // an MN-major operand needs its row count a multiple of 4 for that.
-    bool dl32 = false;
-    if (in_dtype == TF_F32 && BN == 128) {
-        if (K > 0 && K % 32 == 0 && p.vec_a && p.vec_b && ext_ok) {
-            const bool part_m = trans_a == 0 || M % 4 == 0;
-            const bool part_n = trans_b != 0 || N % 4 == 0;
-            p.int_m = part_m ? p.tiles_m : (int)(M / BM);
-            p.int_n = part_n ? p.tiles_n : (int)(N / 128);
-            p.a_bytes = (uint32_t)(ext_a * 4);
-            p.b_bytes = (uint32_t)(ext_b * 4);
-            dl32 = p.int_m * p.int_n > 0;
-            if (!dl32) p.int_m = p.int_n = 0;
+    // fp32: the direct-to-LDS kernel, by 16-byte loads where every operand
+    // row starts on one and holds whole ones, else by 4-byte loads.
+    if (in_dtype == TF_F32 && K > 0 && ext_ok && (reinterpret_cast<uintptr_t>(A) & 3) == 0 &&
+        (reinterpret_cast<uintptr_t>(B) & 3) == 0) {
+        const bool vec = p.vec_a && p.vec_b && ((!a_kmaj && !b_kmaj) || K % 4 == 0) && (a_kmaj || M % 4 == 0) &&
+                         (b_kmaj || N % 4 == 0);
+        const int mode = !vec ? kF32Words : K % kF32K == 0 ? kF32Whole : kF32Tail;
+        p.a_bytes = (uint32_t)(ext_a * 4);
+        p.b_bytes = (uint32_t)(ext_b * 4);
+        p.units_tile = (int)(((K + kF32K - 1) / kF32K) * p.reduce_batch);
+        const F32Plan plan = f32_plan(ncu, M, N, p.units_tile, grid_batch, mode);
+        const int TM = 64 * plan.MI, TN = 64 * plan.NI;
+        p.tiles_m = (int)((M + TM - 1) / TM);
+        p.tiles_n = (int)((N + TN - 1) / TN);
+        const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * grid_batch;
+        TF_REQUIRE(tiles < (1LL << 31), "tf_gemm: too many tiles");
+        p.kb_per_split = (p.units_tile + plan.splits - 1) / plan.splits;
+        const int slices = (p.units_tile + p.kb_per_split - 1) / p.kb_per_split;
+        const int64_t groups = plan.groups ? plan.groups : tiles;
+        p.units_per = (int)(tiles * p.units_tile / groups);
+        p.units_rem = (int)(tiles * p.units_tile % groups);
+        p.tickets = ctx->tickets + tfh::kTicketGemm;
+        if (plan.groups || slices > 1) {
+            const size_t floats = plan.groups ? (size_t)2 * groups * TM * TN : (size_t)slices * M * N;
+            tf_status st = partials_buffer(ctx, floats * sizeof(float), noalloc, &p.partial);
+            if (st != TF_OK) return st;
         }
+        const bool whole = plan.MI + plan.NI == 4 && mode == kF32Whole && !plan.groups && slices == 1;
+        KernelFn fn = whole                           ? pick_f32_whole(a_kmaj, b_kmaj)
+                      : plan.MI + plan.NI == 4 ? pick_f32_dl<2, 2>(a_kmaj, b_kmaj, mode, plan.groups != 0)
+                      : plan.MI == 2           ? pick_f32_dl<2, 1>(a_kmaj, b_kmaj, mode, plan.groups != 0)
+                                               : pick_f32_dl<1, 2>(a_kmaj, b_kmaj, mode, plan.groups != 0);
+        // The whole-tile kernel takes the batch as a grid dimension.
+        const dim3 grid = whole ? dim3((unsigned)(tiles / grid_batch), 1, (unsigned)grid_batch)
+                                : dim3((unsigned)groups, (unsigned)slices);
+        if (whole) p.kb_per_split = p.units_tile;
+        fn<<<grid, kF32DlThreads, 0, ctx->stream>>>(p);
+        tf_status st = tfh::check_launch("gemm_f32_dl_kernel");
+        return st == TF_OK && slices > 1 ? launch_splitk_reduce(ctx, p, slices) : st;
     }
 
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
@@ -3401,21 +3862,6 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         pick_bf16_mid(a_kmaj, b_kmaj, K % 64 != 0)<<<grid, 2 * kThreads, 0, ctx->stream>>>(p);
         st = tfh::check_launch("gemm_bf16_mid_kernel");
         if (st != TF_OK) return st;
-    } else if (dl32) {
-        const int64_t n_int = (int64_t)p.int_m * p.int_n;
-        GemmParams q = p;
-        q.tiles_m = p.int_m;
-        q.tiles_n = p.int_n;
-        dim3 grid((unsigned)n_int, (unsigned)splits, (unsigned)grid_batch);
-        pick_f32_dl(a_kmaj, b_kmaj)<<<grid, kF32DlThreads, 0, ctx->stream>>>(q);
-        st = tfh::check_launch("gemm_f32_dl_kernel");
-        if (st != TF_OK) return st;
-        if (tiles - n_int > 0) {
-            dim3 egrid((unsigned)(tiles - n_int), (unsigned)splits, (unsigned)grid_batch);
-            pick_f32<128>(a_kmaj, b_kmaj)<<<egrid, kThreads, 0, ctx->stream>>>(p);
-            st = tfh::check_launch("gemm_f32_kernel");
-            if (st != TF_OK) return st;
-        }
     } else {
         KernelFn fn = in_dtype == TF_F32 ? (BN == 128 ? pick_f32<128>(a_kmaj, b_kmaj) : pick_f32<64>(a_kmaj, b_kmaj))
                                          : (BN == 128 ? pick_bf16<128>(a_kmaj, b_kmaj) : pick_bf16<64>(a_kmaj, b_kmaj));
@@ -3424,15 +3870,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         st = tfh::check_launch("gemm kernel");
         if (st != TF_OK) return st;
     }
-    if (splits > 1) {
-        if (splits >= 16) {
-            splitk_reduce_wide_kernel<<<(unsigned)((M * N + 15) / 16), 256, 0, ctx->stream>>>(p, splits);
-        } else {
-            dim3 rgrid((unsigned)((N + 1023) / 1024), (unsigned)std::min<int64_t>(M, 65535));
-            splitk_reduce_kernel<<<rgrid, 256, 0, ctx->stream>>>(p, splits);
-        }
-        st = tfh::check_launch("splitk_reduce_kernel");
-    }
+    if (splits > 1) st = launch_splitk_reduce(ctx, p, splits);
     return st;
 }
 

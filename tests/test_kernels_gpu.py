@@ -490,6 +490,61 @@ def test_gemm_bf16_direct_k_tail(ctx, ta, tb, nb, M, N, K, pad):
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("nb,reduce,M,N,K,pad,epi,out_bf16,beta", [
+    (1, False, 129, 257, 2085, 0, "bias_relu", False, 0.0),    # 4-byte loads, K tail, tiles shared by workgroups
+    (1, False, 1001, 1203, 130, 3, "row_bias", True, 0.0),     # 4-byte loads, odd rows of C
+    (1, False, 700, 900, 2100, 0, "bias", False, 0.0),         # 16-byte loads with a K tail
+    (1, False, 64, 2048, 4096, 4, "none", False, 0.5),         # 64-row tiles, beta * C
+    (1, False, 2000, 60, 2304, 0, "row_bias_relu", False, 0.0),  # 64-column tiles
+    (1, False, 300, 200, 20001, 0, "none", False, 0.0),        # few tiles, K in slices
+    (3, False, 520, 516, 600, 8, "bias", True, 0.0),           # independent products
+    (5, True, 64, 576, 1003, 0, "none", False, 0.0),           # batch reduction: the walk wraps after a tail
+    (1, False, 2304, 2176, 64, 0, "none", False, 0.0),         # more tiles than CUs, two k blocks each
+])
+def test_gemm_f32_direct_tiles(ctx, ta, tb, nb, reduce, M, N, K, pad, epi, out_bf16, beta):
+    """The fp32 direct-to-LDS tiles at the edges of their load forms, tile
+    shapes and work splits.  A sum of n fp32 products in any order is off by
+    at most n * 2^-24 of the sum of magnitudes, 1.2e-3 for the longest here in
+    the worst case and about its root (1e-5) in these: RTOL32, and one bf16
+    rounding (2^-8) where C is bf16.  Padding and neighbours hold values that
+    would show in the sums."""
+    import tensors_amd as ta_mod
+    from tensors_amd import _lib, ops
+    lda, ldb = (M if ta else K) + pad, (K if tb else N) + pad
+    a = synth.normal(271 + K, (nb, K if ta else M, lda))
+    b = synth.normal(272 + K, (nb, N if tb else K, ldb))
+    c0 = synth.normal(273, (1 if reduce else nb, M, N))
+    dc = ctx.zeros(c0.shape, ta_mod.BF16) if out_bf16 else ctx.array(c0)
+    rows = epi.startswith("row")
+    bias = None if epi == "none" else synth.normal(274, (M if rows else N,))
+    code = {"none": _lib.TF_EPI_NONE, "bias": _lib.TF_EPI_BIAS, "bias_relu": _lib.TF_EPI_BIAS_RELU,
+            "row_bias": _lib.TF_EPI_ROW_BIAS, "row_bias_relu": _lib.TF_EPI_ROW_BIAS_RELU}[epi]
+    da, db, dbias = ctx.array(a), ctx.array(b), None if bias is None else ctx.array(bias)
+
+    def run():
+        ops.gemm_ex(da, db, dc, M, N, K, lda=lda, ldb=ldb, ldc=N, trans_a=ta, trans_b=tb,
+                    stride_a=a.shape[1] * lda, stride_b=b.shape[1] * ldb, stride_c=M * N, batch=nb,
+                    reduce_batch=reduce, alpha=0.75, beta=beta, epilogue=code, bias=dbias)
+        return dc.numpy()
+
+    prod = [_gemm_truth(a[e][:, :M] if ta else a[e][:, :K], b[e][:, :K] if tb else b[e][:, :N], ta, tb)
+            for e in range(nb)]
+    truth = 0.75 * (sum(prod)[None] if reduce else np.stack(prod)) + beta * c0.astype(np.float64)
+    if bias is not None:
+        truth = truth + (bias[:, None] if rows else bias[None, :]).astype(np.float64)
+    if epi.endswith("relu"):
+        truth = np.maximum(truth, 0.0)
+    got = run()
+    assert_close(ta_mod.bf16_bits_to_f32(got) if out_bf16 else got, truth, 2.0 ** -8 if out_bf16 else RTOL32,
+                 f"f32 direct {nb}x{M}x{N}x{K} {epi}")
+    if beta == 0.0:
+        # The shared tiles' last workgroup adds in a fixed order and leaves
+        # the counters at zero.
+        for _ in range(20):
+            assert_bitexact(run(), got, "repeated")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("nb,reduce,M,N,K,pad,epi,out_bf16,beta", [
     (1, False, 128, 128, 64, 0, "none", False, 0.0),          # one tile, one k block
     (1, False, 8, 16, 8, 8, "bias_relu", False, 0.0),         # a corner of one tile, 56 of 64 k masked
     (1, False, 136, 264, 136, 0, "bias", True, 0.0),          # ragged edges and K tail
