@@ -33,6 +33,11 @@ struct tf_ctx {
     // per-row losses).  Grown on demand from the pool; stream-ordered.
     void* ws = nullptr;
     size_t ws_bytes = 0;
+    // Partial tiles of products whose tiles several workgroups share
+    // (kSharesBytes; allocated by the first such product, held until
+    // shutdown): apart from ws, so that needing them never moves the
+    // workspace that a captured graph refers to.
+    void* shares = nullptr;
     // Block cache in front of the pool (tf_hip_alloc / tf_hip_free): freed
     // blocks wait here by size class and go to the next request of that
     // class, stream-ordered on `stream` like the pool's own reuse.  A pool
@@ -72,6 +77,13 @@ tf_status hip_error(hipError_t e, const char* what);
 
 // Make sure ctx->ws holds at least `bytes`; returns TF_OK or an error.
 tf_status ensure_workspace(tf_ctx* ctx, size_t bytes);
+// Bytes of workspace a launch can count on: while a graph is being captured
+// what is there, otherwise anything.
+inline size_t workspace_limit(const tf_ctx* ctx) { return ctx->capturing ? ctx->ws_bytes : ~size_t(0); }
+// The context's shares, or null where they are not there and cannot be had (a
+// capture in progress, no memory): the caller then does without them.
+constexpr size_t kSharesBytes = size_t(32) << 20;
+float* shares_or_null(tf_ctx* ctx);
 // out[m][n] (row stride ldc) = sum over s < splits of part[s][m][n] in a
 // fixed order (16 split groups, each ascending, combined in a tree).
 tf_status sum_partials(tf_ctx* ctx, const float* part, int64_t splits, int64_t M, int64_t N, float* out, int64_t ldc);

@@ -3511,7 +3511,7 @@ Bf16Plan bf16_plan(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t batch, 
             best.splits = s;
         }
     }
-    if (big_fits) {
+    if (big_fits && (big_splits == 1 || (size_t)big_splits * (size_t)M * (size_t)N * 4 <= partial_limit)) {
         const double t = rounds(kBigTile, big_splits) * (12.0 + 0.0255 * (double)K / big_splits) +
                          (big_splits > 1 ? 4.5 + 0.2 * mb * big_splits : 0.0);
         if (t <= least) best = Bf16Plan{true, big_splits};
@@ -3537,7 +3537,10 @@ struct F32Plan {
     int64_t groups;
     int splits;
 };
-F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t batch, int mode) {
+// `share`: whether workgroups may share tiles; `plane_limit`: bytes of K
+// slices' partials.
+F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t batch, int mode, bool share,
+                 size_t plane_limit) {
     F32Plan best{2, 2, 0, 1};
     double least = 1e300;
     const double unit = mode == kF32Words ? 2.2 : 1.9;
@@ -3556,11 +3559,12 @@ F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t bat
         if (wide) consider(rounds * (10.0 + (mode == kF32Whole ? 1.71 : unit) * (double)kblocks), 0, 1);
         else if (tiles <= ncu) consider(8.0 + unit * 0.56 * (double)kblocks, 0, 1);
         else consider(rounds * (8.0 + unit * (double)kblocks), 0, 1);
-        if (tiles <= tfh::kTicketGemmTiles && units >= 2 * slots && units < (int64_t(1) << 31) && tiles != slots)
+        if (share && tiles <= tfh::kTicketGemmTiles && units >= 2 * slots &&
+            (size_t)2 * slots * 64 * s[0] * 64 * s[1] * 4 <= tfh::kSharesBytes && units < (int64_t(1) << 31) && tiles != slots)
             consider(14.0 + unit * (double)((units + slots - 1) / slots) + (tiles > slots ? 4.0 : 0.0) +
                          0.5 * (double)slots / (double)tiles, slots, 1);
         const int64_t slices = std::min<int64_t>({slots / std::max<int64_t>(tiles, 1), kblocks / 4, 128});
-        if (batch == 1 && slices > 1)
+        if (batch == 1 && slices > 1 && (size_t)slices * (size_t)M * (size_t)N * 4 <= plane_limit)
             consider(15.0 + unit * (double)((kblocks + slices - 1) / slices) +
                          0.35 * (double)slices * (double)M * (double)N * 4e-6, 0, (int)slices);
     }
@@ -3665,7 +3669,7 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     if (in_dtype == TF_BF16 && K > 0 && K % 8 == 0 && p.vec_a && p.vec_b && ext_ok && (trans_a == 0 || M % 8 == 0) &&
         (trans_b != 0 || N % 8 == 0)) {
         const Bf16Plan plan = bf16_plan(ncu, M, N, K * (reduce_batch ? batch : 1), grid_batch, big, splits,
-                                        noalloc ? kNoAllocScratchBytes : ~size_t(0));
+                                        noalloc ? kNoAllocScratchBytes : tfh::workspace_limit(ctx));
         big = plan.big;
         mid = !plan.big;
         splits = plan.splits;
@@ -3783,7 +3787,16 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         p.a_bytes = (uint32_t)(ext_a * 4);
         p.b_bytes = (uint32_t)(ext_b * 4);
         p.units_tile = (int)(((K + kF32K - 1) / kF32K) * p.reduce_batch);
-        const F32Plan plan = f32_plan(ncu, M, N, p.units_tile, grid_batch, mode);
+        const size_t limit = noalloc ? kNoAllocScratchBytes : tfh::workspace_limit(ctx);
+        F32Plan plan = f32_plan(ncu, M, N, p.units_tile, grid_batch, mode, true, limit);
+        if (plan.groups) {
+            if (noalloc) {
+                tf_status st = scratch_address(ctx->device, &p.partial);
+                if (st != TF_OK) return st;
+            } else if (!(p.partial = tfh::shares_or_null(ctx))) {
+                plan = f32_plan(ncu, M, N, p.units_tile, grid_batch, mode, false, limit);
+            }
+        }
         const int TM = 64 * plan.MI, TN = 64 * plan.NI;
         p.tiles_m = (int)((M + TM - 1) / TM);
         p.tiles_n = (int)((N + TN - 1) / TN);
@@ -3795,9 +3808,8 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         p.units_per = (int)(tiles * p.units_tile / groups);
         p.units_rem = (int)(tiles * p.units_tile % groups);
         p.tickets = ctx->tickets + tfh::kTicketGemm;
-        if (plan.groups || slices > 1) {
-            const size_t floats = plan.groups ? (size_t)2 * groups * TM * TN : (size_t)slices * M * N;
-            tf_status st = partials_buffer(ctx, floats * sizeof(float), noalloc, &p.partial);
+        if (slices > 1) {
+            tf_status st = partials_buffer(ctx, (size_t)slices * M * N * sizeof(float), noalloc, &p.partial);
             if (st != TF_OK) return st;
         }
         const bool whole = plan.MI + plan.NI == 4 && mode == kF32Whole && !plan.groups && slices == 1;

@@ -870,13 +870,16 @@ tf_status tf_layernorm_bwd(tf_ctx* ctx, const float* dy, const float* x, const f
                                                                                (int)W, (int)cols, W % 4 == 0);
         return tfh::check_launch("ln_part_strip_kernel");
     }
-    if (const int t = block_threads(cols)) {
+    // (A capture that lacks the room for its partials takes the streamed
+    // kernels below, which need less.)
+    const int64_t nblocks = std::min<int64_t>(rows, std::max<int64_t>(128, std::min<int64_t>(256, rows / 4)));
+    const size_t need = (size_t)nblocks * 2 * cols * sizeof(float);
+    if (const int t = need <= tfh::workspace_limit(ctx) ? block_threads(cols) : 0) {
         // A block a CU: the next row's loads are in flight beside a row's
         // sums, and every block more adds a row of partials (2 x cols,
         // written and read again): 4096 x 4096 takes 42.5 us on 256 blocks,
         // 45.5 on 512; 333 x 5001 16.3 us on 128, 20.2 on 256.
-        const int64_t nblocks = std::min<int64_t>(rows, std::max<int64_t>(128, std::min<int64_t>(256, rows / 4)));
-        tf_status st = tfh::ensure_workspace(ctx, (size_t)nblocks * 2 * cols * sizeof(float));
+        tf_status st = tfh::ensure_workspace(ctx, need);
         if (st != TF_OK) return st;
         float* part = reinterpret_cast<float*>(ctx->ws);
         const bool bvec = vec && row_vec(gamma, cols);

@@ -153,6 +153,15 @@ tf_status ensure_workspace(tf_ctx* ctx, size_t bytes) {
     return TF_OK;
 }
 
+float* shares_or_null(tf_ctx* ctx) {
+    if (!ctx->shares && !ctx->capturing) {
+        void* p = nullptr;
+        if (hipMallocFromPoolAsync(&p, kSharesBytes, ctx->pool, ctx->stream) == hipSuccess) ctx->shares = p;
+        else (void)hipGetLastError();
+    }
+    return static_cast<float*>(ctx->shares);
+}
+
 }  // namespace tfh
 
 extern "C" {
@@ -221,6 +230,7 @@ tf_status tf_hip_shutdown(tf_ctx* ctx) {
         for (auto& kv : ctx->cached)
             for (void* p : kv.second) (void)hipFreeAsync(p, ctx->own_stream);
         if (ctx->ws) (void)hipFreeAsync(ctx->ws, ctx->own_stream);
+        if (ctx->shares) (void)hipFreeAsync(ctx->shares, ctx->own_stream);
         (void)hipStreamSynchronize(ctx->own_stream);
         (void)hipStreamDestroy(ctx->own_stream);
     }

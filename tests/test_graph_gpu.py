@@ -59,6 +59,43 @@ def test_graph_replays_match_eager_calls(ctx):
         call("tf_graph_destroy", g)
 
 
+def test_capture_without_room_for_partials_runs_without_them():
+    """A product that shares tiles between workgroups, or splits K, when run
+    eagerly is captured by a fresh context too, which has no room for the
+    partial sums: it runs unsplit, and eager products that allocate that room
+    afterwards leave the graph valid.  fp32 sums of 100 and bf16 ones of 512
+    products: within 512 * 2^-24 of the sum of magnitudes in any order."""
+    import tensors_amd as ta
+    own = ta.Context(0)
+    try:
+        a, b = synth.normal(1301, (1500, 100)), synth.normal(1302, (100, 1500))
+        h, w = (ta.f32_to_bf16_bits(synth.normal(s, (512, 512))) for s in (1303, 1304))
+        da, db, c = own.array(a), own.array(b), own.zeros((1500, 1500))
+        dh, dw, z = own.array(h, ta.BF16), own.array(w, ta.BF16), own.zeros((512, 512))
+
+        def seq():
+            ops.gemm(da, db, c)
+            ops.gemm(dh, dw, z, trans_a=True)
+
+        want = a.astype(np.float64) @ b.astype(np.float64)
+        zw = ta.bf16_bits_to_f32(h).astype(np.float64).T @ ta.bf16_bits_to_f32(w).astype(np.float64)
+        own.sync()
+        call("tf_graph_begin", own.handle)
+        seq()
+        g = _end(own)
+        try:
+            for r in range(3):
+                call("tf_graph_launch", own.handle, g)
+                for got, ref in ((c, want), (z, zw)):
+                    assert np.abs(got.numpy() - ref).max() < 1e-4 * np.abs(ref).max(), f"replay {r}"
+                seq()                                      # eagerly: the shares are allocated now
+        finally:
+            call("tf_graph_destroy", g)
+    finally:
+        del da, db, c, dh, dw, z
+        own.close()
+
+
 def test_capture_fails_on_a_cache_miss_and_on_sync(ctx):
     call("tf_graph_begin", ctx.handle)
     p = C.c_void_p()
