@@ -330,9 +330,10 @@ tf_status tf_colsum_bf16(tf_ctx* ctx, const void* dy, float* db, int64_t rows, i
  * db[c] = sum_r dz[r, c]: the ReLU backward (autograd/ops/ReluBackward.hpp:22-32)
  * of a ReLU that follows a Linear with bias, fused with that Linear's bias
  * gradient (nn::Linear::forward_relu's backward).  dtype TF_F32 or TF_BF16
- * (dy, x, dz); db is fp32.  dz is bit-identical to tf_relu_bwd and db to
- * tf_colsum / tf_colsum_bf16 of that dz; one pass over dy and x where the
- * column-strip launch applies, else those two calls. */
+ * (dy, x, dz); db is fp32.  dz is bit-identical to tf_relu_bwd, db the
+ * column sums of that dz in a fixed order (within fp32 rounding of tf_colsum /
+ * tf_colsum_bf16); one pass over dy and x where the column-strip launch
+ * applies, else those two calls. */
 tf_status tf_relu_bwd_colsum(tf_ctx* ctx, const void* dy, const void* x, void* dz, float* db, int64_t rows,
                              int64_t cols, int dtype);
 /* C = (A * [mask > 0]) B in fp32, the ReLU backward folded into the load of a

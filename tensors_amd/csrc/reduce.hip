@@ -223,8 +223,32 @@ constexpr int kRcCols = 256;   // columns per strip (64 lanes x 4)
 constexpr int kRcU = 8;        // rows in flight per wave
 constexpr int kRcRows = 128;   // rows per chunk (64 and 256 measured slower at the C5 shapes)
 constexpr int kRcMaxBlocks = 4096;
+// Shorter chunks, down to one batch of loads a wave, where longer ones leave
+// the GPU idle; each halving doubles the chunks that a strip's last block adds
+// (sixteen loads at a time), so it stops at 16 chunks, or 64 below 128 blocks:
+// 512 x 8192 bf16 11.3 -> 8.9 us (128 -> 512 blocks), 512 x 1024 9.5 -> 5.0,
+// 1000 x 1000 fp32 14.3 -> 7.8; 2048 x 2048 fp32 keeps 128 rows (14.9 us; 64
+// rows 15.4, 32 rows 16.8).
+int64_t rc_chunk_rows(int64_t rows, int64_t strips) {
+    int64_t r = kRcRows;
+    auto chunks = [&](int64_t n) { return (rows + n - 1) / n; };
+    while (r > 32 && strips * chunks(r) < 512 && chunks(r / 2) <= (strips * chunks(r) < 128 ? 64 : 16)) r /= 2;
+    return r;
+}
+// Rows that do not start on a whole access, at least this many values: one
+// pass (999 x 1001 fp32 12.7 -> 8.4 us, 100 x 701 10.5 -> 5.4).
+constexpr int64_t kRcScalarMin = 1 << 16;
 
-template <typename T>
+// One value by itself: dz and its value in fp32.
+__device__ __forceinline__ float relu_bwd1(float g, float x, float* dz) { return *dz = g * relu_mask(x); }
+__device__ __forceinline__ float relu_bwd1(uint16_t g, uint16_t x, uint16_t* dz) {
+    return tfd::bf16_to_f32(*dz = tfd::f32_to_bf16(tfd::bf16_to_f32(g) * relu_mask(tfd::bf16_to_f32(x))));
+}
+
+// VEC: 4 consecutive columns a lane in one access.  Otherwise (rows that do
+// not start on such an access) a lane takes columns lane, lane + 64, ... of
+// the strip one by one, four rows in flight.
+template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void relu_bwd_colsum_kernel(const T* __restrict__ dy, const T* __restrict__ x,
                                                               T* __restrict__ dz, float* __restrict__ db,
                                                               float* __restrict__ part, unsigned* __restrict__ tickets,
@@ -234,11 +258,32 @@ __global__ __launch_bounds__(256) void relu_bwd_colsum_kernel(const T* __restric
     __shared__ bool last;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int strip = blockIdx.x, chunk = blockIdx.y;
-    const int c = strip * kRcCols + 4 * lane;
-    const bool on = c < cols;   // cols % 4 == 0: a lane's 4 columns are all in or all out
+    const int c = strip * kRcCols + (VEC ? 4 * lane : lane), cstep = VEC ? 1 : 64;
+    const bool on = c < cols;   // VEC: cols % 4 == 0, so a lane's 4 columns are all in or all out
     const int r0 = chunk * rpc, r1 = min(rows, r0 + rpc);
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (on) {
+    if constexpr (!VEC) {
+        float* a = reinterpret_cast<float*>(&acc);
+        constexpr int U = 4;
+        for (int r = r0 + wave; r < r1; r += 4 * U) {
+            T g[U][4], m[U][4];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    // Past the last row or column: the last one's, not used.
+                    const int64_t off = (int64_t)min(r + 4 * u, r1 - 1) * cols + min(c + 64 * q, cols - 1);
+                    g[u][q] = dy[off];
+                    m[u][q] = x[off];
+                }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    if (r + 4 * u < r1 && c + 64 * q < cols)
+                        a[q] += relu_bwd1(g[u][q], m[u][q], dz + (int64_t)(r + 4 * u) * cols + c + 64 * q);
+        }
+    } else if (on) {
         int r = r0 + wave;
         for (; r + 4 * (kRcU - 1) < r1; r += 4 * kRcU) {
             R4 g[kRcU], m[kRcU];
@@ -266,11 +311,11 @@ __global__ __launch_bounds__(256) void relu_bwd_colsum_kernel(const T* __restric
         const float4 a = red[0][lane], b1 = red[1][lane], c2 = red[2][lane], d = red[3][lane];
         const float sum[4] = {(a.x + b1.x) + (c2.x + d.x), (a.y + b1.y) + (c2.y + d.y), (a.z + b1.z) + (c2.z + d.z),
                               (a.w + b1.w) + (c2.w + d.w)};
-        float* mine = part + ((int64_t)strip * chunks + chunk) * kRcCols + 4 * lane;
+        float* mine = part + ((int64_t)strip * chunks + chunk) * kRcCols + (VEC ? 4 * lane : lane);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if (chunks == 1) db[c + e] = sum[e];
-            else __hip_atomic_store(mine + e, sum[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (chunks > 1) __hip_atomic_store(mine + cstep * e, sum[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            else if (VEC || c + 64 * e < cols) db[c + cstep * e] = sum[e];
         }
     }
     if (chunks == 1) return;
@@ -281,23 +326,21 @@ __global__ __launch_bounds__(256) void relu_bwd_colsum_kernel(const T* __restric
                (unsigned)(chunks - 1);
     __syncthreads();
     if (!last) return;
-    // A thread per column of the strip: the chunks' sums eight loads at a
+    // A thread per column of the strip: the chunks' sums sixteen loads at a
     // time in flight, added in chunk order.
     const int col = strip * kRcCols + threadIdx.x;
     if (col < cols) {
         const float* sp = part + (int64_t)strip * chunks * kRcCols + threadIdx.x;
         float v = 0.0f;
-        int k = 0;
-        for (; k + 8 <= chunks; k += 8) {
-            float t[8];
+        for (int k = 0; k < chunks; k += 16) {
+            float t[16];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                t[u] = __hip_atomic_load(sp + (int64_t)(k + u) * kRcCols, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int u = 0; u < 16; ++u)
+                t[u] = __hip_atomic_load(sp + (int64_t)min(k + u, chunks - 1) * kRcCols, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-            for (int u = 0; u < 8; ++u) v += t[u];
+            for (int u = 0; u < 16; ++u) v += k + u < chunks ? t[u] : 0.0f;
         }
-        for (; k < chunks; ++k)
-            v += __hip_atomic_load(sp + (int64_t)k * kRcCols, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         db[col] = v;
     }
     if (threadIdx.x == 0) __hip_atomic_store(tickets + strip, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -467,17 +510,21 @@ tf_status relu_bwd_colsum_impl(tf_ctx* ctx, const T* dy, const T* x, T* dz, floa
     const bool vec = ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) |
                        reinterpret_cast<uintptr_t>(dz)) & amask) == 0 && cols % 4 == 0;
     const int64_t strips = (cols + kRcCols - 1) / kRcCols;
-    if (vec && strips <= tfh::kTicketColsumStrips) {
-        // Chunks of kRcRows rows, fewer when that would exceed kRcMaxBlocks
-        // blocks.
-        int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((rows + kRcRows - 1) / kRcRows,
+    // Without whole accesses only what is large enough to fill the GPU: small
+    // matrices are faster in the two calls below.
+    if (strips <= tfh::kTicketColsumStrips && (vec || rows * cols >= kRcScalarMin)) {
+        // Chunks of kRcRows rows or shorter, fewer when that would exceed
+        // kRcMaxBlocks blocks.
+        const int64_t chunk_rows = rc_chunk_rows(rows, strips);
+        int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((rows + chunk_rows - 1) / chunk_rows,
                                                                 (kRcMaxBlocks + strips - 1) / strips));
         const int rpc = (int)((rows + chunks - 1) / chunks);
         chunks = (rows + rpc - 1) / rpc;
         TF_REQUIRE(chunks <= 65535, "tf_relu_bwd_colsum: too many row chunks");
         tf_status st = tfh::ensure_workspace(ctx, (size_t)strips * chunks * kRcCols * sizeof(float));
         if (st != TF_OK) return st;
-        relu_bwd_colsum_kernel<T><<<dim3((unsigned)strips, (unsigned)chunks), 256, 0, ctx->stream>>>(
+        auto kernel = vec ? relu_bwd_colsum_kernel<T, true> : relu_bwd_colsum_kernel<T, false>;
+        kernel<<<dim3((unsigned)strips, (unsigned)chunks), 256, 0, ctx->stream>>>(
             dy, x, dz, db, reinterpret_cast<float*>(ctx->ws), ctx->tickets + tfh::kTicketColsum, (int)rows, (int)cols,
             rpc, (int)chunks);
         return tfh::check_launch("relu_bwd_colsum_kernel");

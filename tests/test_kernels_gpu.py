@@ -1113,6 +1113,14 @@ def test_relu_bwd_colsum(ctx, dtype, R, Cc):
     assert_close(db.numpy()[ok], truth[ok], RTOL32, f"relu_bwd_colsum db {dtype} {R}x{Cc} vs float64")
 
 
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("R,Cc", [(999, 1001), (512, 2048), (1, 65537), (3000, 257), (70, 1023), (8200, 8)])
+def test_relu_bwd_colsum_chunks_and_odd_rows(ctx, dtype, R, Cc):
+    """The same checks where the row chunks are short (32 to 128 rows) and
+    where rows do not start on a whole access (a value a lane)."""
+    test_relu_bwd_colsum(ctx, dtype, R, Cc)
+
+
 def test_colsum_zero_rows(ctx):
     ops = _ops()
     db = ctx.array(np.full(7, 3.0, np.float32))
