@@ -207,7 +207,9 @@ tf_status tf_gemm(tf_ctx* ctx, int trans_a, int trans_b,
  * kernels and results as tf_gemm; the split-K partials, which tf_gemm keeps
  * in the context's pool-grown workspace, go to a fixed 64 MiB device array
  * instead (one per GPU, held until the process ends).  A shape whose
- * partials need more is rejected with TF_ERR_INVALID.  Every call on a GPU
+ * partials need more is rejected with TF_ERR_INVALID; bf16 operands whose rows
+ * are not 16-byte loadable and whose packed copies do not fit beside the
+ * partials take the kernels that need no copies (other sum orders).  Every call on a GPU
  * shares that GPU's array: calls that overlap on one GPU (two streams, two
  * threads) race and must be ordered by the caller. */
 tf_status tf_gemm_noalloc(tf_ctx* ctx, int trans_a, int trans_b,

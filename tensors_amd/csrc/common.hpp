@@ -84,6 +84,10 @@ inline size_t workspace_limit(const tf_ctx* ctx) { return ctx->capturing ? ctx->
 // capture in progress, no memory): the caller then does without them.
 constexpr size_t kSharesBytes = size_t(32) << 20;
 float* shares_or_null(tf_ctx* ctx);
+// A temporary for launches on the context's stream, given back with
+// tf_hip_free once they are enqueued; null where there is no memory or, while
+// a graph is being captured, no block of its class at hand.
+void* temp_or_null(tf_ctx* ctx, size_t bytes);
 // out[m][n] (row stride ldc) = sum over s < splits of part[s][m][n] in a
 // fixed order (16 split groups, each ascending, combined in a tree).
 tf_status sum_partials(tf_ctx* ctx, const float* part, int64_t splits, int64_t M, int64_t N, float* out, int64_t ldc);

@@ -3571,6 +3571,88 @@ F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t bat
     return best;
 }
 
+// Copies of bf16 operands whose rows the direct-to-LDS kernels cannot load (not
+// on 16 bytes, or not whole loads long): rows padded with zeros to a multiple
+// of eight.  A pass over the operand at about 3 TB/s, against register-staged
+// tiles at 50 to 200 TF/s (us, NN): 2048 x 3900 x 4000 332 -> 103, 4096 x 8191
+// x 4096 1266 -> 272, 1250 x 1175 x 1218 93 -> 30, 506 x 978 x 2283 41 -> 31,
+// 129 x 2050 x 1030 (just over the limit) 32 -> 27.
+constexpr double kPackMinWork = 1 << 28;   // M * N * K from which it pays
+
+__global__ __launch_bounds__(256) void pack_rows_bf16_kernel(const uint16_t* __restrict__ src, int64_t ld, uint32_t rows,
+                                                             uint32_t len, uint16_t* __restrict__ dst,
+                                                             uint32_t groups) {
+    // Thread: eight values of a row, loaded one by one (any alignment; a
+    // wave's loads cover the same lines), stored together.
+    const uint32_t total = rows * groups;
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const uint32_t row = i / groups, c = 8 * (i - row * groups);
+        const uint16_t* s = src + (int64_t)row * ld + c;
+        uint32_t v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = c + e < len ? s[e] : 0;
+        reinterpret_cast<u32x4*>(dst)[i] = u32x4{v[0] | v[1] << 16, v[2] | v[3] << 16, v[4] | v[5] << 16, v[6] | v[7] << 16};
+    }
+}
+
+// The packed copies of one product, alive until its launches are enqueued.
+struct PackedOperands {
+    const void* a = nullptr;
+    const void* b = nullptr;
+    int64_t lda = 0, ldb = 0;
+    ~PackedOperands() {
+        for (void* t : temp)
+            if (t) (void)tf_hip_free(ctx, t);
+    }
+    // Packs what is given (null: nothing to do), a [rows x len] matrix of
+    // leading dimension ld each.  Leaves a and b null where the room is
+    // lacking.  `partials`: bytes at the start of the fixed scratch that the
+    // product itself uses (tf_gemm_noalloc, which takes the rest of it).
+    tf_status make(tf_ctx* c, bool noalloc, size_t partials, const void* A, int64_t ra, int64_t la, int64_t ld_a,
+                   const void* B, int64_t rb, int64_t lb, int64_t ld_b) {
+        ctx = c;
+        const auto bytes = [](int64_t r, int64_t l) { return (size_t)r * (size_t)((l + 7) / 8) * 16; };
+        const size_t na = A ? bytes(ra, la) : 0, nb = B ? bytes(rb, lb) : 0, lim = size_t(0x7fffffff);
+        if (na > lim || nb > lim) return TF_OK;
+        char* room[2] = {};
+        if (noalloc) {
+            const size_t at = (partials + 255) / 256 * 256, mid = at + (na + 255) / 256 * 256;
+            if (mid + nb > kNoAllocScratchBytes) return TF_OK;
+            float* scratch0 = nullptr;
+            tf_status st = scratch_address(ctx->device, &scratch0);
+            if (st != TF_OK) return st;
+            room[0] = reinterpret_cast<char*>(scratch0) + at;
+            room[1] = reinterpret_cast<char*>(scratch0) + mid;
+        } else {
+            for (int i = 0; i < 2; ++i) {
+                const size_t n = i ? nb : na;
+                if (n == 0) continue;
+                temp[i] = tfh::temp_or_null(ctx, n);
+                if (!temp[i]) return TF_OK;
+                room[i] = static_cast<char*>(temp[i]);
+            }
+        }
+        tf_status st = TF_OK;
+        if (A) st = launch(A, ra, la, ld_a, room[0], a, lda);
+        if (B && st == TF_OK) st = launch(B, rb, lb, ld_b, room[1], b, ldb);
+        return st;
+    }
+
+private:
+    tf_ctx* ctx = nullptr;
+    void* temp[2] = {};
+    tf_status launch(const void* src, int64_t rows, int64_t len, int64_t ld, char* dst, const void*& out,
+                     int64_t& out_ld) {
+        const int64_t groups = (len + 7) / 8;
+        pack_rows_bf16_kernel<<<tfd::grid_for(rows * groups, 2), 256, 0, ctx->stream>>>(
+            static_cast<const uint16_t*>(src), ld, (uint32_t)rows, (uint32_t)len, reinterpret_cast<uint16_t*>(dst),
+            (uint32_t)groups);
+        out = dst;
+        out_ld = 8 * groups;
+        return tfh::check_launch("pack_rows_bf16_kernel");
+    }
+};
+
 // Grid of the small-product kernel for an M x N x K product: 32 x 32 tiles
 // and enough chunk groups for ~256 blocks, at most 32 per tile (the last
 // block adds them up), each of >= 1 chunk of 64 k.  False when the product
@@ -3661,15 +3743,34 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
     }
     // The direct-to-LDS kernels need 16-byte loadable operands, a K of whole
     // 16-byte loads and extents that fit the buffer descriptor (taken as int).
-    const int64_t ext_a = trans_a ? (K - 1) * lda + M : (M - 1) * lda + K;
-    const int64_t ext_b = trans_b ? (N - 1) * ldb + K : (K - 1) * ldb + N;
-    const bool ext_ok = ext_a * esz <= (int64_t)0x7fffffff && ext_b * esz <= (int64_t)0x7fffffff;
+    int64_t ext_a = trans_a ? (K - 1) * lda + M : (M - 1) * lda + K;
+    int64_t ext_b = trans_b ? (N - 1) * ldb + K : (K - 1) * ldb + N;
+    const auto ext_fits = [&](int64_t a, int64_t b) { return a * esz <= 0x7fffffff && b * esz <= 0x7fffffff; };
+    const bool ext_ok = ext_fits(ext_a, ext_b);
     p.vec_a = aligned16(A) && (lda % vec_elems == 0) && (stride_a % vec_elems == 0);
     p.vec_b = aligned16(B) && (ldb % vec_elems == 0) && (stride_b % vec_elems == 0);
-    if (in_dtype == TF_BF16 && K > 0 && K % 8 == 0 && p.vec_a && p.vec_b && ext_ok && (trans_a == 0 || M % 8 == 0) &&
-        (trans_b != 0 || N % 8 == 0)) {
-        const Bf16Plan plan = bf16_plan(ncu, M, N, K * (reduce_batch ? batch : 1), grid_batch, big, splits,
-                                        noalloc ? kNoAllocScratchBytes : tfh::workspace_limit(ctx));
+    // A K-major operand's last load holds whole values past K unless K % 8 ==
+    // 0; an MN-major one's k rows are loaded or left out one by one.
+    const bool a_direct = p.vec_a && (a_kmaj ? K % 8 == 0 : M % 8 == 0);
+    const bool b_direct = p.vec_b && (b_kmaj ? K % 8 == 0 : N % 8 == 0);
+    bool direct16 = in_dtype == TF_BF16 && K > 0 && a_direct && b_direct && ext_ok;
+    const auto plan16 = [&](size_t limit) {
+        return bf16_plan(ncu, M, N, K * (reduce_batch ? batch : 1), grid_batch, big, splits, limit);
+    };
+    const size_t limit16 = noalloc ? kNoAllocScratchBytes : tfh::workspace_limit(ctx);
+    PackedOperands packed;
+    if (in_dtype == TF_BF16 && !direct16 && batch == 1 && (double)M * (double)N * (double)K >= kPackMinWork) {
+        const Bf16Plan plan = plan16(limit16);
+        const size_t partials = plan.splits > 1 ? (size_t)plan.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+        tf_status st = packed.make(ctx, noalloc, partials, a_direct ? nullptr : A, a_kmaj ? M : K, a_kmaj ? K : M, lda,
+                                   b_direct ? nullptr : B, b_kmaj ? N : K, b_kmaj ? K : N, ldb);
+        if (st != TF_OK) return st;
+        if (packed.a) { p.A = packed.a; p.lda = packed.lda; p.vec_a = 1; ext_a = (a_kmaj ? M : K) * packed.lda; }
+        if (packed.b) { p.B = packed.b; p.ldb = packed.ldb; p.vec_b = 1; ext_b = (b_kmaj ? N : K) * packed.ldb; }
+        direct16 = (a_direct || packed.a) && (b_direct || packed.b) && ext_fits(ext_a, ext_b);
+    }
+    if (direct16) {
+        const Bf16Plan plan = plan16(limit16);
         big = plan.big;
         mid = !plan.big;
         splits = plan.splits;
@@ -3762,8 +3863,9 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         // kernels count splits in 64-deep blocks, the last one partial when
         // K % 64 != 0, so their split boundaries agree) and each operand's
         // extent fits the buffer descriptor.
-        const int64_t k_unit = kBf16Kernel >= 1 ? 8 : 64;   // the four-wave kernel has no K tail
-        const bool direct = K > 0 && K % k_unit == 0 && p.vec_a && p.vec_b && ext_ok;
+        // (The four-wave kernel has no K tail.)
+        const bool direct = kBf16Kernel >= 1 ? direct16 || (K > 0 && K % 8 == 0 && p.vec_a && p.vec_b && ext_ok)
+                                             : K > 0 && K % 64 == 0 && p.vec_a && p.vec_b && ext_ok;
         p.a_bytes = direct ? (uint32_t)(ext_a * esz) : 0u;
         p.b_bytes = direct ? (uint32_t)(ext_b * esz) : 0u;
         // Partial tiles at the M / N edges are fine for the direct kernel:
@@ -3771,8 +3873,8 @@ tf_status gemm_impl(tf_ctx* ctx, int trans_a, int trans_b, int64_t M, int64_t N,
         // rows past M or N inside it only feed outputs that are not stored.
         // An MN-major operand needs its row count a multiple of 8 for that,
         // so no 16-byte load straddles the end of its extent.
-        const bool part_m = trans_a == 0 || M % 8 == 0;
-        const bool part_n = trans_b != 0 || N % 8 == 0;
+        const bool part_m = trans_a == 0 || M % 8 == 0 || packed.a != nullptr;
+        const bool part_n = trans_b != 0 || N % 8 == 0 || packed.b != nullptr;
         p.int_m = direct ? (int)(part_m ? (M + kBigTile - 1) / kBigTile : M / kBigTile) : 0;
         p.int_n = direct ? (int)(part_n ? (N + kBigTile - 1) / kBigTile : N / kBigTile) : 0;
     }

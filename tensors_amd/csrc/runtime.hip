@@ -471,3 +471,22 @@ tf_status tf_hip_event_destroy(void* event) {
 }
 
 }  // extern "C"
+
+namespace tfh {
+
+void* temp_or_null(tf_ctx* ctx, size_t bytes) {
+    if (ctx->capturing) {
+        std::lock_guard<std::mutex> lock(ctx->cache_mu);
+        const size_t cls = size_class(bytes);
+        const auto held = [&](const std::unordered_map<size_t, std::vector<void*>>& m) {
+            const auto it = m.find(cls);
+            return it != m.end() && !it->second.empty();
+        };
+        if (!held(ctx->capture_free) && !held(ctx->cached)) return nullptr;
+    }
+    void* p = nullptr;
+    return tf_hip_alloc(ctx, bytes, &p) == TF_OK ? p : nullptr;
+}
+
+}  // namespace tfh
+

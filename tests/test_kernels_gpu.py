@@ -489,6 +489,42 @@ def test_gemm_bf16_direct_k_tail(ctx, ta, tb, nb, M, N, K, pad):
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("M,N,K,pad,shift", [
+    (515, 1027, 513, 0, 0),      # odd in every extent
+    (1024, 512, 516, 0, 0),      # whole rows but for K % 8
+    (512, 1040, 520, 3, 0),      # whole extents, odd leading dimensions
+    (768, 768, 512, 0, 1),       # whole extents, bases one value off
+    (4100, 4099, 260, 0, 0),     # large tiles, K tail
+])
+def test_gemm_bf16_unaligned_operands(ctx, ta, tb, M, N, K, pad, shift):
+    """bf16 operands whose rows are not 16-byte loadable: packed copies in
+    front of the direct-to-LDS tiles.  Sums of up to 520 exact products in
+    fp32: within 520 * 2^-24 = 3e-5 of the sum of magnitudes, RTOL32.
+    tf_gemm_noalloc takes the same kernels where the copies fit its scratch:
+    the same bits."""
+    import tensors_amd as ta_mod
+    from tensors_amd import _lib
+    from tensors_amd._lib import call
+    lda, ldb = (M if ta else K) + pad, (K if tb else N) + pad
+    a_shape, b_shape = (K if ta else M, lda), (N if tb else K, ldb)
+    a16 = ta_mod.f32_to_bf16_bits(synth.normal(281 + K, a_shape))
+    b16 = ta_mod.f32_to_bf16_bits(synth.normal(282 + K, b_shape))
+    a, b = ta_mod.bf16_bits_to_f32(a16), ta_mod.bf16_bits_to_f32(b16)
+    # `shift` values of something else before each operand.
+    da = ctx.array(np.concatenate([np.full(shift, 0x7FC0, np.uint16), a16.ravel()]), ta_mod.BF16)
+    db = ctx.array(np.concatenate([np.full(shift, 0x7FC0, np.uint16), b16.ravel()]), ta_mod.BF16)
+    out = []
+    for entry in ("tf_gemm", "tf_gemm_noalloc"):
+        dc = ctx.zeros((M, N))
+        call(entry, ctx.handle, int(ta), int(tb), M, N, K, 1.0, da.ptr + 2 * shift, lda, db.ptr + 2 * shift, ldb, 0.0,
+             dc.ptr, N, _lib.TF_BF16, _lib.TF_F32, _lib.TF_EPI_NONE, None)
+        out.append(dc.numpy())
+    truth = _gemm_truth(a[:, :M] if ta else a[:, :K], b[:, :K] if tb else b[:, :N], ta, tb)
+    assert_close(out[0], truth, RTOL32, f"bf16 unaligned ta={ta} tb={tb} {M}x{N}x{K} pad={pad} shift={shift}")
+    assert_bitexact(out[1], out[0], "tf_gemm_noalloc")
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("nb,reduce,M,N,K,pad,epi,out_bf16,beta", [
     (1, False, 129, 257, 2085, 0, "bias_relu", False, 0.0),    # 4-byte loads, K tail, tiles shared by workgroups
     (1, False, 1001, 1203, 130, 3, "row_bias", True, 0.0),     # 4-byte loads, odd rows of C
