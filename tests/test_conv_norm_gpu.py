@@ -466,6 +466,28 @@ def test_col2im_checks_out_extent(ctx):
 
 
 
+# Planes whose column rows do not fit the LDS (more than 16384 values): one to
+# five taps an axis, non-square extents and strides, few planes and many, and
+# eleven taps (the element form).  The same adds in the same order as the
+# host's loop over (ki, kj): the same bits.
+@pytest.mark.parametrize("N,Cc,H,W,kH,kW,s,p", [
+    (2, 3, 80, 81, 3, 3, (1, 1), (1, 1)), (1, 2, 150, 131, 1, 1, (1, 1), (0, 0)), (3, 1, 120, 77, 5, 5, (2, 1), (2, 0)),
+    (2, 2, 90, 90, 7, 3, (3, 1), (2, 3)), (1, 1, 70, 70, 9, 9, (2, 2), (4, 4)), (300, 1, 64, 65, 3, 3, (1, 1), (1, 1)),
+    (1, 1, 60, 60, 11, 11, (1, 1), (5, 5)),
+])
+def test_col2im_large_planes_bitexact(ctx, N, Cc, H, W, kH, kW, s, p):
+    ops = _ops()
+    oh, ow = ops.conv_out(H, kH, s[0], p[0], 1), ops.conv_out(W, kW, s[1], p[1], 1)
+    col = synth.normal(221 + H, (N, Cc, kH, kW, oh, ow))
+    want = np.zeros((N, Cc, H + 2 * p[0] + s[0], W + 2 * p[1] + s[1]), np.float32)
+    for ki in range(kH):
+        for kj in range(kW):
+            want[:, :, ki:ki + oh * s[0]:s[0], kj:kj + ow * s[1]:s[1]] += col[:, :, ki, kj]
+    dx = ctx.array(np.full((N, Cc, H, W), 7.0, np.float32))
+    ops.col2im(ctx.array(col), dx, kH, kW, stride=s, pad=p)
+    assert_bitexact(dx.numpy(), np.ascontiguousarray(want[:, :, p[0]:p[0] + H, p[1]:p[1] + W]), "col2im")
+
+
 RELU_CASES = [
     (128, 3, 32, 32, 32, 3, 1, 1, 1),      # C4 conv1
     (128, 32, 32, 32, 64, 3, 2, 1, 1),     # C4 conv2
