@@ -3523,12 +3523,13 @@ Bf16Plan bf16_plan(int64_t ncu, int64_t M, int64_t N, int64_t K, int64_t batch, 
 // workgroups that share its units evenly (0: one per tile and K slice) or
 // `splits` K slices.  Estimated in us from measured products (ncu = 256):
 //   128 x 128 whole tiles 10 + 1.71 a 32-deep block and round;
-//   shared units 14 + 1.9 a unit (2.2 with 4-byte loads), 4 more where the
-//   workgroups run over several tiles, and 0.5 per workgroup on a tile;
+//   shared units 14 + 1.9 a unit (2.2 with 4-byte loads), 4.5 for each tile
+//   that a workgroup runs over, and 0.5 per workgroup on a tile;
 //   K slices 15 + 1.9 a block, and 0.35 a MB of partials;
 //   the 64-wide tiles, two to a CU, take as long a unit as a 128 x 128 one
-//   does (half the work a unit at twice the units in flight), and 1.02 us
-//   alone on their CU.
+//   does (half the work a unit at twice the units in flight) and 5.5 a round,
+//   and 1.02 us a unit alone on their CU: 576 x 3136 x 64 over 32 images 128 us
+//   on 64 x 128 tiles, 139 on shared 128 x 128 ones.
 // Against the register-staged 128 x 64 kernel and its K split (us): 999 x 3072
 // x 1001 150-158 -> 70, 999 x 1001 x 3072 85-120 -> 58-68, 1000 x 3072 x 1024
 // 110-212 -> 60, 512 x 4096 x 2048 86-97 -> 69, 64 x 4096 x 4096 56-115 -> 35.
@@ -3558,10 +3559,11 @@ F32Plan f32_plan(int64_t ncu, int64_t M, int64_t N, int64_t kblocks, int64_t bat
         const double rounds = (double)((tiles + slots - 1) / slots);
         if (wide) consider(rounds * (10.0 + (mode == kF32Whole ? 1.71 : unit) * (double)kblocks), 0, 1);
         else if (tiles <= ncu) consider(8.0 + unit * 0.56 * (double)kblocks, 0, 1);
-        else consider(rounds * (8.0 + unit * (double)kblocks), 0, 1);
+        else consider(rounds * (5.5 + unit * (double)kblocks), 0, 1);
         if (share && tiles <= tfh::kTicketGemmTiles && units >= 2 * slots &&
             (size_t)2 * slots * 64 * s[0] * 64 * s[1] * 4 <= tfh::kSharesBytes && units < (int64_t(1) << 31) && tiles != slots)
-            consider(14.0 + unit * (double)((units + slots - 1) / slots) + (tiles > slots ? 4.0 : 0.0) +
+            consider(14.0 + unit * (double)((units + slots - 1) / slots) +
+                         (tiles > slots ? 4.5 * (double)tiles / (double)slots : 0.0) +
                          0.5 * (double)slots / (double)tiles, slots, 1);
         const int64_t slices = std::min<int64_t>({slots / std::max<int64_t>(tiles, 1), kblocks / 4, 128});
         if (batch == 1 && slices > 1 && (size_t)slices * (size_t)M * (size_t)N * 4 <= plane_limit)
