@@ -54,6 +54,7 @@ struct tf_ctx {
     // destroyed, so a replay's temporaries are never handed to other work.
     bool capturing = false;
     bool capture_failed = false;  // a call failed while capturing
+    int graphs = 0;               // captured graphs not yet destroyed
     std::unordered_map<size_t, std::vector<void*>> capture_free;
     // Blocks allocated during the current capture (the graph's kernels hold
     // their addresses), and, after tf_graph_end, those of them still live,
@@ -77,9 +78,12 @@ tf_status hip_error(hipError_t e, const char* what);
 
 // Make sure ctx->ws holds at least `bytes`; returns TF_OK or an error.
 tf_status ensure_workspace(tf_ctx* ctx, size_t bytes);
-// Bytes of workspace a launch can count on: while a graph is being captured
-// what is there, otherwise anything.
-inline size_t workspace_limit(const tf_ctx* ctx) { return ctx->capturing ? ctx->ws_bytes : ~size_t(0); }
+// Bytes of workspace a launch that has another form should take: what is there
+// while a graph is being captured (it may not grow) or exists (growing moves
+// it, and the graph could not be launched again), otherwise anything.
+inline size_t workspace_limit(const tf_ctx* ctx) {
+    return ctx->capturing || ctx->graphs > 0 ? ctx->ws_bytes : ~size_t(0);
+}
 // The context's shares, or null where they are not there and cannot be had (a
 // capture in progress, no memory): the caller then does without them.
 constexpr size_t kSharesBytes = size_t(32) << 20;

@@ -132,6 +132,7 @@ tf_status tf_graph_end(tf_ctx* ctx, tf_graph** out) {
     g->graph = graph;
     g->exec = exec;
     g->ws = ctx->ws;
+    ++ctx->graphs;
     g->held = std::move(held);
     {
         // Blocks allocated during capture and still live: a later free hands
@@ -172,6 +173,7 @@ tf_status tf_graph_destroy(tf_graph* g) {
         for (auto it = ctx->graph_owned.begin(); it != ctx->graph_owned.end();)
             it = it->second == &g->held ? ctx->graph_owned.erase(it) : std::next(it);
     }
+    --ctx->graphs;
     delete g;
     if (e1 != hipSuccess) return tfh::hip_error(e1, "tf_graph_destroy: hipGraphExecDestroy");
     if (e2 != hipSuccess) return tfh::hip_error(e2, "tf_graph_destroy: hipGraphDestroy");

@@ -870,8 +870,9 @@ tf_status tf_layernorm_bwd(tf_ctx* ctx, const float* dy, const float* x, const f
                                                                                (int)W, (int)cols, W % 4 == 0);
         return tfh::check_launch("ln_part_strip_kernel");
     }
-    // (A capture that lacks the room for its partials takes the streamed
-    // kernels below, which need less.)
+    // (A capture that lacks the room for its partials, or a call beside a graph
+    // that they would invalidate, takes the streamed kernels below, which need
+    // less.)
     const int64_t nblocks = std::min<int64_t>(rows, std::max<int64_t>(128, std::min<int64_t>(256, rows / 4)));
     const size_t need = (size_t)nblocks * 2 * cols * sizeof(float);
     if (const int t = need <= tfh::workspace_limit(ctx) ? block_threads(cols) : 0) {

@@ -510,18 +510,21 @@ tf_status relu_bwd_colsum_impl(tf_ctx* ctx, const T* dy, const T* x, T* dz, floa
     const bool vec = ((reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(x) |
                        reinterpret_cast<uintptr_t>(dz)) & amask) == 0 && cols % 4 == 0;
     const int64_t strips = (cols + kRcCols - 1) / kRcCols;
-    // Without whole accesses only what is large enough to fill the GPU: small
-    // matrices are faster in the two calls below.
-    if (strips <= tfh::kTicketColsumStrips && (vec || rows * cols >= kRcScalarMin)) {
-        // Chunks of kRcRows rows or shorter, fewer when that would exceed
-        // kRcMaxBlocks blocks.
-        const int64_t chunk_rows = rc_chunk_rows(rows, strips);
-        int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((rows + chunk_rows - 1) / chunk_rows,
-                                                                (kRcMaxBlocks + strips - 1) / strips));
-        const int rpc = (int)((rows + chunks - 1) / chunks);
-        chunks = (rows + rpc - 1) / rpc;
+    // Chunks of kRcRows rows or shorter, fewer when that would exceed
+    // kRcMaxBlocks blocks.
+    const int64_t chunk_rows = rc_chunk_rows(rows, strips);
+    int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((rows + chunk_rows - 1) / chunk_rows,
+                                                            (kRcMaxBlocks + strips - 1) / strips));
+    const int rpc = (int)((rows + chunks - 1) / chunks);
+    chunks = (rows + rpc - 1) / rpc;
+    const size_t need = (size_t)strips * chunks * kRcCols * sizeof(float);
+    // Without whole accesses only what is large enough to fill the GPU (small
+    // matrices are faster in the two calls below) and, beside a captured
+    // graph, what the workspace at hand holds: the two calls need less.
+    if (strips <= tfh::kTicketColsumStrips &&
+        (vec || (rows * cols >= kRcScalarMin && need <= tfh::workspace_limit(ctx)))) {
         TF_REQUIRE(chunks <= 65535, "tf_relu_bwd_colsum: too many row chunks");
-        tf_status st = tfh::ensure_workspace(ctx, (size_t)strips * chunks * kRcCols * sizeof(float));
+        tf_status st = tfh::ensure_workspace(ctx, need);
         if (st != TF_OK) return st;
         auto kernel = vec ? relu_bwd_colsum_kernel<T, true> : relu_bwd_colsum_kernel<T, false>;
         kernel<<<dim3((unsigned)strips, (unsigned)chunks), 256, 0, ctx->stream>>>(

@@ -96,6 +96,76 @@ def test_capture_without_room_for_partials_runs_without_them():
         own.close()
 
 
+def test_relu_bwd_colsum_capture_without_workspace():
+    """Rows that do not start on a whole access, in a context that has no
+    workspace yet: the capture takes the form that needs none.  dz is exact;
+    column sums of 32768 values: within 32768 * 2^-24 of the sum of magnitudes."""
+    import tensors_amd as ta
+    own = ta.Context(0)
+    try:
+        rows, cols = 32768, 2
+        dy, x = synth.normal(1305, (rows, cols)), synth.normal(1306, (rows, cols))
+        ddy, dx, dz, db = own.array(dy), own.array(x), own.zeros((rows, cols)), own.zeros((cols,))
+        want = dy * (x > 0)
+        own.sync()
+        call("tf_graph_begin", own.handle)
+        ops.relu_bwd_colsum(ddy, dx, dz, db)
+        g = _end(own)
+        try:
+            for r in range(3):
+                call("tf_graph_launch", own.handle, g)
+                assert np.array_equal(dz.numpy(), want), f"replay {r}"
+                bound = rows * 2.0 ** -24 * np.abs(want).astype(np.float64).sum(0)
+                assert (np.abs(db.numpy() - want.astype(np.float64).sum(0)) <= bound).all(), f"replay {r}"
+                ops.relu_bwd_colsum(ddy, dx, dz, db)
+        finally:
+            call("tf_graph_destroy", g)
+    finally:
+        del ddy, dx, dz, db
+        own.close()
+
+
+def test_layernorm_bwd_beside_a_graph_leaves_it_valid():
+    """A LayerNorm backward whose block-per-row form wants more workspace than a
+    captured graph found runs beside that graph without moving it.  Sums of
+    4096 terms in dx, 256 in dgamma and dbeta: far within 4096 * 2^-24 of the
+    largest value."""
+    import tensors_amd as ta
+    own = ta.Context(0)
+    try:
+        rows, cols = 256, 4096
+        x, dy = synth.normal(1307, (rows, cols)), synth.normal(1308, (rows, cols))
+        gamma = synth.normal(1309, (cols,)) + np.float32(1)
+        dx_, ddy, dg, db0 = own.array(x), own.array(dy), own.array(gamma), own.zeros((cols,))
+        y, mean, rstd = own.zeros((rows, cols)), own.zeros((rows,)), own.zeros((rows,))
+        gx, gg, gb = own.zeros((rows, cols)), own.zeros((cols,)), own.zeros((cols,))
+        s = own.zeros((cols,))
+        ops.colsum(dx_, s)                                  # a workspace of the smallest size
+        ops.layernorm_fwd(dx_, dg, db0, y, mean, rstd)
+        own.sync()
+        call("tf_graph_begin", own.handle)
+        ops.colsum(dx_, s)
+        g = _end(own)
+        try:
+            x64, dy64 = x.astype(np.float64), dy.astype(np.float64)
+            r = 1 / np.sqrt(x64.var(1, keepdims=True) + 1e-5)
+            xh = (x64 - x64.mean(1, keepdims=True)) * r
+            d = dy64 * gamma
+            want = (r * (d - d.mean(1, keepdims=True) - xh * (d * xh).mean(1, keepdims=True)),
+                    (dy64 * xh).sum(0), dy64.sum(0))
+            for i in range(2):
+                ops.layernorm_bwd(ddy, dx_, dg, mean, rstd, gx, gg, gb)
+                for got, ref in zip((gx, gg, gb), want):
+                    assert np.abs(got.numpy() - ref).max() <= 4096 * 2.0 ** -24 * np.abs(ref).max()
+                call("tf_graph_launch", own.handle, g)
+                assert np.abs(s.numpy() - x64.sum(0)).max() <= 256 * 2.0 ** -24 * np.abs(x64).sum(0).max()
+        finally:
+            call("tf_graph_destroy", g)
+    finally:
+        del dx_, ddy, dg, db0, y, mean, rstd, gx, gg, gb, s
+        own.close()
+
+
 def test_capture_fails_on_a_cache_miss_and_on_sync(ctx):
     call("tf_graph_begin", ctx.handle)
     p = C.c_void_p()
